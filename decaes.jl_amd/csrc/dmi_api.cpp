@@ -76,7 +76,7 @@ int no_capture(dmi_ctx *c, const char *name) {
 // launch counters and the per-workgroup slots of the voxel kernel.
 struct RunBufs {
     dmi_host::GridPtrs g;
-    int64_t *vox;
+    int64_t *vox, *redo;  // the voxel list, and as much room for the voxels the register-resident kernel leaves
     int64_t vox_cap;
     unsigned *counter;
     unsigned long long *counters;
@@ -112,6 +112,7 @@ int run_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, con
     bool tune = o->schedule == DMI_SCHED_AUTO && cands.size() > 1 && !dmi_host::schedule_lookup(o, sched);
     bool launched = false;
     double tune_ms = 0.0;
+    int64_t last = 0;  // voxels of the last chunk's launch, whose second launch waits for its count
     for (int64_t v0 = 0; v0 < V; v0 += rb.vox_cap) {
         const int64_t v1 = std::min<int64_t>(V, v0 + rb.vox_cap);
         HIPCHECK(c, dmi::launch_fill(rb.counter, sizeof(unsigned), 0u, c->stream));
@@ -132,8 +133,8 @@ int run_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, con
                     dmi::T2mapParams ps = p;
                     dmi_host::apply_schedule(ps, s);
                     HIPCHECK(c, hipEventRecord(c->ev[1], c->stream));
-                    int rc = dmi_host::t2map_launch_raw(c->err, ps, rb.vox + done, cnt, rb.counter, rb.counters,
-                                                        rb.status, rb.slots, rb.slot_doubles, c->num_cu, c->stream);
+                    int rc = dmi_host::t2map_launch_raw(c->err, ps, rb.vox + done, cnt, rb.counter, rb.counters, rb.status,
+                                                        rb.redo, rb.slots, rb.slot_doubles, c->num_cu, c->stream);
                     if (rc) return rc;
                     HIPCHECK(c, hipEventRecord(c->ev[2], c->stream));
                     HIPCHECK(c, hipEventSynchronize(c->ev[2]));
@@ -151,21 +152,33 @@ int run_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, con
         if (!launched) HIPCHECK(c, hipEventRecord(c->ev[1], c->stream));
         launched = true;
         dmi_host::apply_schedule(p, sched);
-        c->stats.lds_rows = std::min(p.rl, p.mw);
+        c->stats.lds_rows = p.rs ? 0 : std::min(p.rl, p.mw);
         c->stats.workgroups_per_cu = sched.per_cu;
         int rc = dmi_host::t2map_launch_raw(c->err, p, rb.vox + done, nvox - done, rb.counter, rb.counters, rb.status,
-                                            rb.slots, rb.slot_doubles, c->num_cu, c->stream);
+                                            rb.redo, rb.slots, rb.slot_doubles, c->num_cu, c->stream, v1 < V);
         if (rc) return rc;
+        last = (v1 == V && p.rs) ? nvox - done : 0;
     }
     unsigned long long cnt[4] = {0, 0, 0, 0};
-    int status = 0;
-    if (launched) {
-        HIPCHECK(c, hipEventRecord(c->ev[2], c->stream));
-        HIPCHECK(c, hipMemcpyAsync(cnt, rb.counters, sizeof cnt, hipMemcpyDeviceToHost, c->stream));
-        HIPCHECK(c, hipMemcpyAsync(&status, rb.status, sizeof status, hipMemcpyDeviceToHost, c->stream));
+    auto finish = [&](unsigned *left) -> int {
+        if (launched) {
+            HIPCHECK(c, hipEventRecord(c->ev[2], c->stream));
+            HIPCHECK(c, hipMemcpyAsync(cnt, rb.counters, sizeof cnt, hipMemcpyDeviceToHost, c->stream));
+            if (left) HIPCHECK(c, hipMemcpyAsync(left, rb.counter + 2, sizeof *left, hipMemcpyDeviceToHost, c->stream));
+        }
+        HIPCHECK(c, hipEventRecord(c->ev[3], c->stream));
+        HIPCHECK(c, hipEventSynchronize(c->ev[3]));
+        return DMI_OK;
+    };
+    // the host reads the tallies here anyway, so the second launch is made only for voxels that need it
+    unsigned left = 0;
+    int rc1 = finish(last > 0 ? &left : nullptr);
+    if (rc1) return rc1;
+    if (left) {
+        rc1 = dmi_host::t2map_launch_redo(c->err, p, last, rb.counter, rb.counters, rb.status, rb.redo, rb.slots, rb.slot_doubles,
+                                          c->num_cu, c->stream);
+        if (rc1 || (rc1 = finish(nullptr))) return rc1;
     }
-    HIPCHECK(c, hipEventRecord(c->ev[3], c->stream));
-    HIPCHECK(c, hipEventSynchronize(c->ev[3]));
     float kms = 0, tms = 0;
     if (launched) HIPCHECK(c, hipEventElapsedTime(&kms, c->ev[1], c->ev[2]));
     HIPCHECK(c, hipEventElapsedTime(&tms, c->ev[0], c->ev[3]));
@@ -175,7 +188,6 @@ int run_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, con
     c->stats.voxels_failed = (int64_t)cnt[3];
     c->stats.kernel_ms = kms + tune_ms;
     c->stats.total_ms = tms;
-    (void)status;
     return DMI_OK;
 }
 
@@ -199,13 +211,13 @@ int record_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, 
     int rc = dmi_host::t2map_schedule(c->err, o, sched);
     if (rc) return rc;
     dmi_host::apply_schedule(p, sched);
-    unsigned *count = rb.counter, *work = rb.counter + 1;
+    unsigned *count = rb.counter;
     p.nvox_dev = count;
     for (int64_t v0 = 0; v0 < V; v0 += rb.vox_cap) {
         const int64_t v1 = std::min<int64_t>(V, v0 + rb.vox_cap);
         HIPCHECK(c, dmi::launch_fill(count, sizeof(unsigned), 0u, c->stream));
         HIPCHECK(c, dmi::launch_select(d_image, v0, v1, o->Threshold, rb.vox, count, c->stream));
-        rc = dmi_host::t2map_launch_raw(c->err, p, rb.vox, v1 - v0, work, rb.counters, rb.status, rb.slots,
+        rc = dmi_host::t2map_launch_raw(c->err, p, rb.vox, v1 - v0, rb.counter, rb.counters, rb.status, rb.redo, rb.slots,
                                         rb.slot_doubles, c->num_cu, c->stream);
         if (rc) return rc;
     }
@@ -225,7 +237,7 @@ int run_t2map(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, const 
     HIPCHECK(c, hipEventRecord(c->ev[0], c->stream));
     rc = c->grids.ensure(c->err, o, c->stream);
     if (rc) return rc;
-    HIPCHECK(c, c->vox.ensure(sizeof(int64_t) * std::max<int64_t>(V, 1)));
+    HIPCHECK(c, c->vox.ensure(2 * sizeof(int64_t) * std::max<int64_t>(V, 1)));
     HIPCHECK(c, c->lb.counter.ensure(sizeof(unsigned) * 4));
     HIPCHECK(c, c->lb.counters.ensure(sizeof(unsigned long long) * 4));
     HIPCHECK(c, c->lb.status.ensure(sizeof(int) * 4));
@@ -238,7 +250,8 @@ int run_t2map(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, const 
         slot_doubles = std::max<int64_t>(slot_doubles, dmi::t2map_slot_doubles(o->nTE, o->nT2, s.rl >= o->nTE + o->nT2 ? 0 : s.gld) *
                                                            std::max<int64_t>(1, std::min<int64_t>((int64_t)c->num_cu * std::max(s.per_cu, 1), V)));
     HIPCHECK(c, c->lb.scratch.ensure(sizeof(double) * (size_t)slot_doubles));
-    RunBufs rb{c->grids.ptrs(), c->vox.as<int64_t>(), std::max<int64_t>(V, 1), c->lb.counter.as<unsigned>(),
+    RunBufs rb{c->grids.ptrs(), c->vox.as<int64_t>(), c->vox.as<int64_t>() + std::max<int64_t>(V, 1),
+               std::max<int64_t>(V, 1), c->lb.counter.as<unsigned>(),
                c->lb.counters.as<unsigned long long>(), c->lb.status.as<int>(), c->lb.scratch.as<double>(), slot_doubles};
     return run_t2map_on(c, d_image, o, d_alpha_in, d, rb);
 }
@@ -272,7 +285,7 @@ int run_t2map_host_chunks(dmi_ctx *c, const double *image, const dmi_t2map_opts 
     if (rc) return rc;
     if (!c->copy_stream) HIPCHECK(c, hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
     hipStream_t cs = c->copy_stream;
-    HIPCHECK(c, c->vox.ensure(sizeof(int64_t) * C));
+    HIPCHECK(c, c->vox.ensure(2 * sizeof(int64_t) * C));
     HIPCHECK(c, c->lb.counter.ensure(sizeof(unsigned) * 4));
     HIPCHECK(c, c->lb.counters.ensure(sizeof(unsigned long long) * 4));
     HIPCHECK(c, c->lb.status.ensure(sizeof(int) * 4));
@@ -297,7 +310,7 @@ int run_t2map_host_chunks(dmi_ctx *c, const double *image, const dmi_t2map_opts 
         for (int i = 0; i < 12; ++i)
             if (hp[i]) HIPCHECK(c, c->pout[b][i].ensure(sizeof(double) * (size_t)(C * rows[i])));
     }
-    RunBufs rb{c->grids.ptrs(), c->vox.as<int64_t>(), C, c->lb.counter.as<unsigned>(),
+    RunBufs rb{c->grids.ptrs(), c->vox.as<int64_t>(), c->vox.as<int64_t>() + C, C, c->lb.counter.as<unsigned>(),
                c->lb.counters.as<unsigned long long>(), c->lb.status.as<int>(), c->lb.scratch.as<double>(), slot_doubles};
     unsigned *cnt = c->pcnt.as<unsigned>();
     auto span = [&](int64_t k, int64_t &v0, int64_t &len) { v0 = k * C; len = std::min<int64_t>(C, V - v0); };
@@ -383,7 +396,7 @@ int run_t2map_host_chunks(dmi_ctx *c, const double *image, const dmi_t2map_opts 
             dmi_host::apply_schedule(p, sched);
             p.nvox_dev = cnt + k;
             HIPCHECK(c, dmi::launch_select(c->pimg[b].as<double>(), 0, len, o->Threshold, rb.vox, cnt + k, c->stream));
-            r = dmi_host::t2map_launch_raw(c->err, p, rb.vox, len, rb.counter + 1, rb.counters, rb.status, rb.slots,
+            r = dmi_host::t2map_launch_raw(c->err, p, rb.vox, len, rb.counter, rb.counters, rb.status, rb.redo, rb.slots,
                                            rb.slot_doubles, c->num_cu, c->stream);
             if (r) return r;
             HIPCHECK(c, hipEventRecord(ev.done[b], c->stream));
@@ -428,7 +441,7 @@ int run_t2map_host_chunks(dmi_ctx *c, const double *image, const dmi_t2map_opts 
     c->stats.voxels_failed = (int64_t)tot[3];
     c->stats.kernel_ms = kms0 + kms;
     c->stats.total_ms = tms;
-    c->stats.lds_rows = std::min(sched.rl, m + n);
+    c->stats.lds_rows = sched.rs ? 0 : std::min(sched.rl, m + n);
     c->stats.workgroups_per_cu = sched.per_cu;
     return DMI_OK;
 }
@@ -462,6 +475,7 @@ int run_t2map_noalloc(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o
     rb.status = reinterpret_cast<int *>(S + 4);                     // S[4, 6)
     rb.counter = reinterpret_cast<unsigned *>(S + 6);               // S[6, 8)
     rb.vox = reinterpret_cast<int64_t *>(S + dmi::kNoAllocOffVox);
+    rb.redo = reinterpret_cast<int64_t *>(S + dmi::kNoAllocOffRedo);
     rb.vox_cap = dmi::kNoAllocVox;
     rb.slots = S + dmi::kNoAllocOffSlots;
     rb.slot_doubles = dmi::kNoAllocSlots;

@@ -219,7 +219,7 @@ void Grids::release() {
 }
 
 void LaunchBufs::release() {
-    for (DevBuf *b : {&counter, &counters, &status, &scratch}) b->release();
+    for (DevBuf *b : {&counter, &counters, &status, &scratch, &redo}) b->release();
 }
 
 dmi::T2mapParams t2map_params(const dmi_t2map_opts *o, const GridPtrs &g, const double *d_image, const double *d_alpha,
@@ -235,6 +235,7 @@ dmi::T2mapParams t2map_params(const dmi_t2map_opts *o, const GridPtrs &g, const 
     p.mw = m + n;
     p.rl = p.lda;  // all rows in LDS unless a schedule says otherwise
     p.gld = 0;
+    p.rs = 0;
     p.save_resnorm = o->SaveResidualNorm; p.save_decaycurve = o->SaveDecayCurve;
     p.save_regparam = o->SaveRegParam; p.save_basis = o->SaveNNLSBasis;
     p.legacy = o->legacy != 0;
@@ -251,6 +252,8 @@ dmi::T2mapParams t2map_params(const dmi_t2map_opts *o, const GridPtrs &g, const 
     p.AsT = fixed ? nullptr : g.AsT;
     p.dAsT = fixed ? nullptr : g.dAsT;
     p.Afixed = fixed ? g.AsT : nullptr;
+    p.As = fixed ? nullptr : g.As;
+    p.AfixedR = fixed ? g.As : nullptr;
     p.alpha_in = d_alpha;
     p.dist = d->dist; p.gdn = d->gdn; p.ggm = d->ggm; p.gva = d->gva; p.fnr = d->fnr; p.snr = d->snr; p.alpha = d->alpha;
     p.resnorm = o->SaveResidualNorm ? d->resnorm : nullptr;
@@ -261,14 +264,28 @@ dmi::T2mapParams t2map_params(const dmi_t2map_opts *o, const GridPtrs &g, const 
     return p;
 }
 
-int t2map_launch_raw(std::string &err, dmi::T2mapParams p, const int64_t *d_vox, int64_t nvox, unsigned *counter,
-                     unsigned long long *counters, int *status, double *slots, int64_t slot_doubles, int num_cu,
-                     hipStream_t s) {
-    if (nvox <= 0) return DMI_OK;
-    const size_t lds = dmi::t2map_lds_bytes(p.m, p.n, p.lda, p.K, p.legacy);
-    int per_cu = 0;
-    DMI_HIP(err, dmi::t2map_occupancy(p.reg, p.legacy, &per_cu, lds, p.rl < p.mw));
+// Workgroups per CU of the voxel kernel in `p`, and its LDS per workgroup.
+static int voxel_occupancy(std::string &err, const dmi::T2mapParams &p, int &per_cu, size_t &lds) {
+    per_cu = 0;
+    if (p.rs) {
+        lds = sizeof(double) * (size_t)dmi::reg_layout(p.m, p.n, p.reg == DMI_REG_GCV).total;
+        DMI_HIP(err, dmi::t2map_occupancy_reg(p.rs, p.reg, &per_cu, lds));
+    } else {
+        lds = dmi::t2map_lds_bytes(p.m, p.n, p.lda, p.K, p.legacy);
+        DMI_HIP(err, dmi::t2map_occupancy(p.reg, p.legacy, &per_cu, lds, p.rl < p.mw));
+    }
     if (per_cu < 1) return errorf(err, DMI_EUNSUPPORTED, "voxel kernel does not fit on a CU (LDS %zu bytes)", lds);
+    return DMI_OK;
+}
+
+int t2map_launch_raw(std::string &err, dmi::T2mapParams p, const int64_t *d_vox, int64_t nvox, unsigned *counter,
+                     unsigned long long *counters, int *status, int64_t *redo, double *slots, int64_t slot_doubles,
+                     int num_cu, hipStream_t s, bool with_redo) {
+    if (nvox <= 0) return DMI_OK;
+    int per_cu = 0;
+    size_t lds = 0;
+    int rc = voxel_occupancy(err, p, per_cu, lds);
+    if (rc) return rc;
     p.slot_stride = dmi::t2map_slot_doubles(p.m, p.n, p.gld);
     const int64_t fit = slot_doubles / p.slot_stride;
     if (fit < 1) return errorf(err, DMI_ECAPACITY, "scratch of %lld doubles holds no voxel slot of %lld doubles",
@@ -277,10 +294,36 @@ int t2map_launch_raw(std::string &err, dmi::T2mapParams p, const int64_t *d_vox,
     p.scratch = slots;
     p.vox = d_vox;
     p.nvox = nvox;
-    p.counter = counter;
+    p.counter = counter + 1;
     p.counters = counters;
     p.status = status;
-    DMI_HIP(err, dmi::launch_fill(counter, sizeof(unsigned), 0u, s));
+    p.redo = redo;
+    p.redo_count = counter + 2;
+    DMI_HIP(err, dmi::launch_fill(counter + 1, 3 * sizeof(unsigned), 0u, s));
+    DMI_HIP(err, dmi::launch_t2map(p, grid, lds, s));
+    return p.rs && with_redo ? t2map_launch_redo(err, p, nvox, counter, counters, status, redo, slots, slot_doubles, num_cu, s)
+                             : DMI_OK;
+}
+
+int t2map_launch_redo(std::string &err, dmi::T2mapParams p, int64_t nvox, unsigned *counter, unsigned long long *counters,
+                      int *status, int64_t *redo, double *slots, int64_t slot_doubles, int num_cu, hipStream_t s) {
+    if (p.reg == DMI_REG_NONE) return DMI_OK;  // its solves have at most m rows, which the class holds
+    p.rs = 0;
+    p.lda = p.rl = dmi::t2map_lda(p.m, p.n);
+    p.gld = 0;
+    p.scratch = slots;
+    p.slot_stride = dmi::t2map_slot_doubles(p.m, p.n, 0);
+    p.vox = redo;
+    p.nvox = nvox;
+    p.nvox_dev = counter + 2;
+    p.counter = counter + 3;
+    p.counters = counters;
+    p.status = status;
+    int per_cu = 0;
+    size_t lds = 0;
+    const int rc = voxel_occupancy(err, p, per_cu, lds);
+    if (rc) return rc;
+    const int grid = (int)std::min<int64_t>(std::min<int64_t>((int64_t)num_cu * per_cu, nvox), slot_doubles / p.slot_stride);
     DMI_HIP(err, dmi::launch_t2map(p, grid, lds, s));
     return DMI_OK;
 }
@@ -291,18 +334,36 @@ int t2map_launch(std::string &err, dmi::T2mapParams p, const int64_t *d_vox, int
     DMI_HIP(err, lb.counter.ensure(sizeof(unsigned) * 4));
     DMI_HIP(err, lb.counters.ensure(sizeof(unsigned long long) * 4));
     DMI_HIP(err, lb.status.ensure(sizeof(int) * 4));
-    const size_t lds = dmi::t2map_lds_bytes(p.m, p.n, p.lda, p.K, p.legacy);
+    if (p.rs) DMI_HIP(err, lb.redo.ensure(sizeof(int64_t) * (size_t)nvox));
     int per_cu = 0;
-    DMI_HIP(err, dmi::t2map_occupancy(p.reg, p.legacy, &per_cu, lds, p.rl < p.mw));
-    if (per_cu < 1) return errorf(err, DMI_EUNSUPPORTED, "voxel kernel does not fit on a CU (LDS %zu bytes)", lds);
+    size_t lds = 0;
+    const int rc = voxel_occupancy(err, p, per_cu, lds);
+    if (rc) return rc;
     const int64_t grid = std::min<int64_t>((int64_t)num_cu * per_cu, nvox);
     const int64_t slot_doubles = dmi::t2map_slot_doubles(p.m, p.n, p.gld) * grid;
     DMI_HIP(err, lb.scratch.ensure(sizeof(double) * (size_t)slot_doubles));
     return t2map_launch_raw(err, p, d_vox, nvox, lb.counter.as<unsigned>(), lb.counters.as<unsigned long long>(),
-                            lb.status.as<int>(), lb.scratch.as<double>(), slot_doubles, num_cu, s);
+                            lb.status.as<int>(), lb.redo.as<int64_t>(), lb.scratch.as<double>(), slot_doubles, num_cu, s);
 }
 
+static int memory_schedules(std::string &err, const dmi_t2map_opts *o, std::vector<Schedule> &out);
+
 int t2map_schedules(std::string &err, const dmi_t2map_opts *o, std::vector<Schedule> &out) {
+    int rc = memory_schedules(err, o, out);
+    if (rc || o->schedule != DMI_SCHED_AUTO || o->legacy) return rc;
+    Schedule r = out.front();  // all rows outside the slot
+    r.rs = dmi::t2map_reg_class(o->nTE, o->Reg);
+    if (!r.rs) return DMI_OK;
+    const size_t lds = sizeof(double) * (size_t)dmi::reg_layout(o->nTE, o->nT2, o->Reg == DMI_REG_GCV).total;
+    DMI_HIP(err, dmi::t2map_occupancy_reg(r.rs, o->Reg, &r.per_cu, lds));
+    if (r.per_cu < 1) return DMI_OK;
+    if (out.size() > 1) out.erase(out.begin(), out.end() - 1);
+    else out.clear();
+    out.insert(out.begin(), r);
+    return DMI_OK;
+}
+
+static int memory_schedules(std::string &err, const dmi_t2map_opts *o, std::vector<Schedule> &out) {
     out.clear();
     const int m = o->nTE, n = o->nT2, K = std::isnan(o->SetFlipAngle) ? o->nRefAngles : 1;
     Schedule full;
@@ -374,6 +435,7 @@ void apply_schedule(dmi::T2mapParams &p, const Schedule &s) {
     p.lda = s.lda;
     p.rl = s.rl;
     p.gld = s.rl >= p.mw ? 0 : s.gld;
+    p.rs = s.rs;
 }
 
 int t2part_prepare(std::string &err, const dmi_t2part_opts *o, std::vector<double> &lg, std::vector<double> &wts,

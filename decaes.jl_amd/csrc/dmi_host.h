@@ -87,7 +87,7 @@ struct Grids {
 
 // Per-launch device state of the voxel kernel: the work counter, tallies, status flags, scratch slots.
 struct LaunchBufs {
-    DevBuf counter, counters, status, scratch;
+    DevBuf counter, counters, status, scratch, redo;
     void release();
 };
 
@@ -104,9 +104,13 @@ int validate_outputs(std::string &err, const dmi_t2map_opts *o, const dmi_t2map_
 // (rows [rl, m + n) live in the workgroup's global slot with column stride gld) and the workgroups that fit a CU.
 struct Schedule {
     int lda = 0, rl = 0, gld = 0, per_cu = 0;
+    int rs = 0;  // register-resident solves (a size class of dmi_internal.h); 0: memory-resident
 };
-// Candidates for these options: the all-LDS schedule first, then, for the Tikhonov-regularized methods (whose
-// workspace has m + n rows), split schedules with the largest LDS part that fits one and two more workgroups per CU.
+// Candidates for these options. Automatic: the register-resident schedule where its size classes hold the train, and, for
+// the Tikhonov-regularized methods, the split schedule with the most workgroups per CU to be measured against it.
+// Otherwise (and for an explicit memory-resident choice): the all-LDS schedule first, then, for the
+// Tikhonov-regularized methods (whose workspace has m + n rows), split schedules with the largest LDS part that fits
+// one and two more workgroups per CU.
 int t2map_schedules(std::string &err, const dmi_t2map_opts *o, std::vector<Schedule> &out);
 // The process-wide choice measured for these sizes and method (false if none yet).
 bool schedule_lookup(const dmi_t2map_opts *o, Schedule &s);
@@ -120,15 +124,22 @@ void apply_schedule(dmi::T2mapParams &p, const Schedule &s);
 dmi::T2mapParams t2map_params(const dmi_t2map_opts *o, const GridPtrs &g, const double *d_image, const double *d_alpha,
                               const dmi_t2map_out *d);
 
-// Launches the voxel kernel on voxels d_vox[0, nvox) of the request in `p` (asynchronous on `s`). Zeroes the
-// work counter; tallies and status accumulate into lb.counters / lb.status until the caller clears them.
+// Launches the voxel kernel on voxels d_vox[0, nvox) of the request in `p` (asynchronous on `s`), and after a
+// register-resident one the memory-resident kernel on the voxels that one left (none as a rule: it then ends at
+// once). Zeroes the work counters; tallies and status accumulate into lb.counters / lb.status until the caller clears them.
 int t2map_launch(std::string &err, dmi::T2mapParams p, const int64_t *d_vox, int64_t nvox, LaunchBufs &lb,
                  int num_cu, hipStream_t s);
-// The same launch on caller-provided device memory: the work counter (zeroed here by a fill kernel), the tallies and
-// status words, and `slot_doubles` doubles of per-workgroup slots, which cap the persistent grid.
+// The same launch on caller-provided device memory: `counter`, four words of which [1] (the work counter), [2] and [3]
+// (the voxels left, and the work counter of their launch) are zeroed here by a fill kernel, the tallies and status
+// words, `redo`, room for nvox voxels, and `slot_doubles` doubles of per-workgroup slots, which cap the persistent grid.
 int t2map_launch_raw(std::string &err, dmi::T2mapParams p, const int64_t *d_vox, int64_t nvox, unsigned *counter,
-                     unsigned long long *counters, int *status, double *slots, int64_t slot_doubles, int num_cu,
-                     hipStream_t s);
+                     unsigned long long *counters, int *status, int64_t *redo, double *slots, int64_t slot_doubles,
+                     int num_cu, hipStream_t s, bool with_redo = true);
+// The second launch of the above by itself (for a caller that passes with_redo = false and reads counter[2] first): the
+// memory-resident kernel, every workspace row in LDS, on the voxels that a register-resident launch left in `redo`.
+// counter[2] is read on the device; nvox bounds it. The slots are free again, as the launches follow each other.
+int t2map_launch_redo(std::string &err, dmi::T2mapParams p, int64_t nvox, unsigned *counter, unsigned long long *counters,
+                      int *status, int64_t *redo, double *slots, int64_t slot_doubles, int num_cu, hipStream_t s);
 
 // T2partSEcorr window ranges, log-T2 values and sigmoid weights (src/T2partSEcorr.jl:143-164).
 int t2part_prepare(std::string &err, const dmi_t2part_opts *o, std::vector<double> &lg, std::vector<double> &wts,

@@ -35,7 +35,8 @@ constexpr int64_t kNoAllocSlots = 5242880;                                   // 
 constexpr int64_t kNoAllocOffGrid = kNoAllocHeader;
 constexpr int64_t kNoAllocOffBasis = kNoAllocOffGrid + kNoAllocGrid;
 constexpr int64_t kNoAllocOffVox = kNoAllocOffBasis + 4 * kNoAllocBasis;
-constexpr int64_t kNoAllocOffSlots = kNoAllocOffVox + kNoAllocVox;
+constexpr int64_t kNoAllocOffRedo = kNoAllocOffVox + kNoAllocVox;                // the chunk's voxels left to the second kernel
+constexpr int64_t kNoAllocOffSlots = kNoAllocOffRedo + kNoAllocVox;
 constexpr int64_t kNoAllocDoubles = kNoAllocOffSlots + kNoAllocSlots;
 constexpr int kNoAllocMaxDevices = 64;
 
@@ -63,6 +64,7 @@ struct T2mapParams {
     int fp32;             // 1: FP32 EPG recursion for the voxel basis (mixed precision)
     int lda, mw;          // workspace: mw = m + n rows, column-major; rows [0, rl) in LDS with column stride lda
     int rl, gld;          // rows [rl, mw) in the workgroup's global slot, column stride gld (rl >= mw: all in LDS)
+    int rs;               // register-resident solves with rs rows per lane (a size class), or 0: memory-resident
     int save_resnorm, save_decaycurve, save_regparam, save_basis;
     int legacy;           // legacy = true: spline surrogate for the flip angle, chi2 doubling search
     int64_t V;            // voxels in the volume
@@ -78,6 +80,10 @@ struct T2mapParams {
     const double *AsT;    // K grid bases, n columns of stride basis_ld(m) each
     const double *dAsT;   // d/dalpha, same layout
     const double *Afixed; // the SetFlipAngle basis, n columns of stride basis_ld(m)
+    const double *As;     // K grid bases, row-major m x n (the register-resident kernel solves on these)
+    const double *AfixedR;// the SetFlipAngle basis, row-major m x n
+    int64_t *redo;        // register-resident kernel: voxels left to the memory-resident one
+    unsigned int *redo_count;
     const double *alpha_in;
     double *scratch;      // per-workgroup slots
     int64_t slot_stride;  // doubles per slot
@@ -95,6 +101,31 @@ struct T2partParams {
     const double *dist;
     double *sfr, *sgm, *mfr, *mgm;
 };
+
+// LDS of one register-resident workgroup (dmi_nnls_reg.h), offsets and total in doubles: the solution x at 0, the
+// right-hand side, the Tikhonov cache's mu, norms and residuals, and the solver's region: the triangular factor packed
+// by column (position j's rows [0, j] at T + j (j + 1) / 2), a column in transit, three vectors of kRegStage rows. GCV's Gram
+// matrix (odd column stride) takes the region between solves.
+constexpr int kRegStage = 144;
+struct RegLayout {
+    int b, c, T, tmp, stg, total;
+};
+__host__ __device__ inline RegLayout reg_layout(int m, int n, bool gram) {
+    RegLayout l;
+    const int ne = (n + 1) & ~1, N = m < n ? m : n;
+    l.b = ne;
+    l.c = l.b + ((m + n + 1) & ~1);
+    l.T = l.c + 3 * kTikhCache;
+    l.tmp = l.T + ((n * (n + 1) / 2 + 1) & ~1);
+    l.stg = l.tmp + ne;
+    l.total = l.stg + 3 * kRegStage;
+    const int g = l.T + ((N * (N | 1) + 1) & ~1);
+    if (gram && l.total < g) l.total = g;
+    // the triangular solve reads 64 rows from the start of every column
+    const int r = l.T + n * (n - 1) / 2 + 64;
+    if (l.total < r) l.total = r;
+    return l;
+}
 
 int t2map_lda(int m, int n);
 // LDS of one voxel workgroup; K (the flip-angle grid size of the launch) takes no LDS; legacy adds the spline knots
@@ -121,5 +152,19 @@ hipError_t t2map_occupancy(int reg, int legacy, int *blocks_per_cu, size_t lds, 
 // the voxel kernel of the split schedule, from dmi_kernels_split.hip (launch_t2map calls it when p.rl < p.mw)
 hipError_t launch_t2map_split(const T2mapParams &p, int grid, size_t lds, hipStream_t s);
 hipError_t t2map_occupancy_split(int reg, int legacy, int *blocks_per_cu, size_t lds);
+// the register-resident voxel kernel of size class S (kRegClasses), one unit per class from dmi_kernels_reg.hip
+// Size classes of the register-resident kernel. A Tikhonov solve's window holds the m rows and the appended rows whose
+// columns have left the active set again; it had at most 13 of those beyond m in 60,000 solves of the benchmark shapes
+// (99.9%: 11), and up to 3 registers are lost to the window's alignment, hence m + 16 rows. Solves without
+// regularization have m rows. A solve that outgrows its class sends the voxel to the memory-resident kernel.
+constexpr int kRegClasses[] = {48, 64, 72, 80};
+inline int t2map_reg_class(int m, int reg) {
+    for (int s : kRegClasses)
+        if (s >= m + (reg == 0 ? 0 : 16)) return s;
+    return 0;
+}
+hipError_t t2map_occupancy_reg(int rs, int reg, int *blocks_per_cu, size_t lds);
+template <int S> hipError_t launch_t2map_reg(const T2mapParams &p, int grid, size_t lds, hipStream_t s);
+template <int S> hipError_t t2map_reg_occupancy(int reg, int *blocks_per_cu, size_t lds);
 
 }  // namespace dmi

@@ -17,9 +17,16 @@
 // (the slot branches of the split schedule compile away) and the host launchers; dmi_kernels_split.hip includes it
 // with DMI_SPLIT_TU = 1 to build only the voxel kernel for the split schedule, whose rows beyond an LDS cutoff live in
 // the workgroup's global slot. The instrumented build (DMI_PHASE_PROFILE) is one unit with the split branches kept.
+// dmi_kernels_reg.hip includes it once per size class (DMI_REG_S registers rows) to build the register-resident voxel
+// kernel (dmi_nnls_reg.h) and its launcher.
 #ifndef DMI_SPLIT_TU
 #define DMI_SPLIT_TU 0
 #endif
+#ifndef DMI_REG_S
+#define DMI_REG_S 0
+#endif
+// the unit that holds every other kernel and the host launchers
+#define DMI_MAIN_TU (!DMI_SPLIT_TU && !DMI_REG_S)
 #if DMI_SPLIT_TU || defined(DMI_PHASE_PROFILE)
 #define DMI_SLOT_ROWS 1
 #else
@@ -28,6 +35,7 @@
 #include <hip/hip_runtime.h>
 #include <mutex>
 #include <type_traits>
+#include <utility>
 
 #include <cfloat>
 #include <climits>
@@ -547,7 +555,7 @@ __global__ void fill_kernel(unsigned int *p, int64_t nwords, unsigned int v) {
 // each device holds for the life of the process. Host code never passes `scratch` itself to a kernel: it takes
 // the device's own address of the array once with hipGetSymbolAddress (noalloc_scratch below).
 // ------------------------------------------------------------------------------------------------
-#if !DMI_SPLIT_TU
+#if DMI_MAIN_TU
 static __device__ __align__(256) double scratch[kNoAllocDoubles];
 #endif
 
@@ -586,6 +594,22 @@ struct Wave {
     bool failed;  // this voxel gets no outputs (a per-voxel cache overflowed)
 
     __device__ __forceinline__ ldbl &Aat(int i, int j) { return A[j * lda + i]; }
+    // The basis the solves read, by element, and the strides (column, row) the voxel's basis is written with.
+    static constexpr bool kRowMajor = false;
+    __device__ __forceinline__ double basis(int i, int j) const { return A0[j * basis_ld(m) + i]; }
+    __device__ __forceinline__ int basis_cs() const { return basis_ld(m); }
+    __device__ __forceinline__ int basis_rs() const { return 1; }
+    // GCV's Gram matrix: rows [m, m + N) of columns [0, N) of the workspace (lda >= m + n leaves the room), formed
+    // from the basis copied into rows [0, m).
+    __device__ __forceinline__ void gram_begin() {
+        load_basis(A0);
+        basis_wait();
+        __syncthreads();
+    }
+    __device__ __forceinline__ double gram_basis(int i, int j) { return Aat(i, j); }
+    __device__ __forceinline__ ldbl &gram_at(int r, int c) { return A[c * lda + m + r]; }
+    __device__ __forceinline__ bool redo() const { return false; }
+    __device__ __forceinline__ void begin_voxel() {}
     // row i of column j wherever it lives (i < rl: LDS, else the global slot); per-lane rows may differ
     __device__ __forceinline__ double Aget(int i, int j) {
         return (!DMI_SLOT_ROWS || i < rl) ? (double)A[j * lda + i] : (double)G[j * gld + (i - rl)];
@@ -1242,6 +1266,10 @@ struct Wave {
     }
 };
 
+#if DMI_REG_S
+#include "dmi_nnls_reg.h"
+#endif
+
 // --------------------------------- scalar optimizers (src/optimization.jl) ---------------------------------
 // bracket_root_monotonic (:191-219)
 template <class F> __device__ __forceinline__ void bracket_root_monotonic(F &&f, double a, double delta, double dilate, double mono,
@@ -1479,7 +1507,7 @@ __device__ __forceinline__ void fprota(double cs, double sn, double &a, double &
 // point i + 1, x increasing). Knots go to W.spt, coefficients to W.spc; returns the knot count n = np + k + 1.
 // Lane j - 1 holds row j of the band triangle (4 entries) and of the rotated right-hand side; every rotation reads
 // its row with readlane, computes in all lanes alike, and the owner keeps the result.
-__device__ int spline_fit(Wave &W, double xv, double yv, int np, int &k_out) {
+template <class Wv> __device__ int spline_fit(Wv &W, double xv, double yv, int np, int &k_out) {
     const int L = W.L;
     const int k = min(3, np - 1), k1 = k + 1, n = np + k1, nk1 = np, k3 = k / 2;
     ldbl *t1 = W.spt - 1;
@@ -1549,7 +1577,7 @@ __device__ int spline_fit(Wave &W, double xv, double yv, int np, int &k_out) {
 // reference's scan with strict '<' keeps it (a NaN first value is never replaced). Lane L scans a contiguous block
 // of samples; the interval search starts where the lane's previous sample left it (the samples increase, so this
 // is the interval splev finds from t(k+1)).
-__device__ void spline_scan(Wave &W, int k, int n, bool root, double v, double &xo, double &yo) {
+template <class Wv> __device__ void spline_scan(Wv &W, int k, int n, bool root, double v, double &xo, double &yo) {
     const int L = W.L, k1 = k + 1, nk1 = n - k1;
     const ldbl *t1 = W.spt - 1, *c1p = W.spc - 1;
     const JlRange r = jl_range(rfl(t1[k1]), 0.001, rfl(t1[n - k]));
@@ -1594,7 +1622,7 @@ __device__ void spline_scan(Wave &W, int k, int n, bool root, double v, double &
 // ------------------------------------ regularization (src/lsqnonneg.jl) ------------------------------------
 // lsqnonneg_chi2! with method :brent (:504-593)
 // (legacy: method :legacy, :521-532, with chi2_search_from_minimum)
-__device__ __forceinline__ void reg_chi2(Wave &W, double chi2_target, bool legacy, double &mu_out, double &chi2_out) {
+template <class Wv> __device__ __forceinline__ void reg_chi2(Wv &W, double chi2_target, bool legacy, double &mu_out, double &chi2_out) {
     int ns;
     double res2_min = W.plain_solve_res2(ns);
     if (res2_min == 0 || ns == 0) {
@@ -1664,7 +1692,7 @@ __device__ __forceinline__ void reg_chi2(Wave &W, double chi2_target, bool legac
 }
 
 // lsqnonneg_mdp! (:700-747)
-__device__ __forceinline__ void reg_mdp(Wave &W, double delta, double &mu_out, double &chi2_out) {
+template <class Wv> __device__ __forceinline__ void reg_mdp(Wv &W, double delta, double &mu_out, double &chi2_out) {
     int ns;
     double res2_min = W.plain_solve_res2(ns);
     if (W.L < W.n) W.xf[W.L] = W.x[W.L];
@@ -1712,19 +1740,17 @@ __device__ __forceinline__ void reg_mdp(Wave &W, double delta, double &mu_out, d
 // calls LAPACK dgesdd (src/utils.jl:96-134); here: Gram matrix of the smaller side, Householder
 // tridiagonalization, then Sturm-sequence bisection, one eigenvalue per lane. Absolute accuracy is
 // eps * ||A||^2, far below the mu^2 >= exp(-16) scale at which gcv_dof uses them.
-__device__ __forceinline__ void gram_eigs(Wave &W, double &lam_lane, int &N) {
-    const int m = W.m, n = W.n, L = W.L, lda = W.lda;
+template <class Wv> __device__ __forceinline__ void gram_eigs(Wv &W, double &lam_lane, int &N) {
+    const int m = W.m, n = W.n, L = W.L;
     DMI_PT0();
-    W.load_basis(W.A0);
-    W.basis_wait();
-    __syncthreads();
+    W.gram_begin();
     N = min(m, n);
-    // N x N Gram matrix at rows [m, m + N) of columns [0, N) (lda >= m + n leaves the room), built with FP64
+    // N x N Gram matrix in LDS (the wave type's gram_at), built with FP64
     // MFMA 16x16x4 blocks: G = A^T A when m >= n, A A^T otherwise. For block (R, C) and k-step s, lane l supplies
     // X[l % 16][s + l / 16] and Y[s + l / 16][l % 16]; the result lane l, register r is D[4r + l / 16][l % 16].
     // Only blocks with R <= C are formed and each value is stored at (row, col) and (col, row), so G is exactly
     // symmetric.
-    auto G = [&](int r, int c) -> ldbl & { return W.A[c * lda + m + r]; };
+    auto G = [&](int r, int c) -> ldbl & { return W.gram_at(r, c); };
     {
         typedef double d4 __attribute__((ext_vector_type(4)));
         const int NB = (N + 15) / 16, K = (m >= n) ? m : n;
@@ -1738,11 +1764,11 @@ __device__ __forceinline__ void gram_eigs(Wave &W, double &lam_lane, int &N) {
                     double a = 0.0, bb = 0.0;
                     if (k < K) {
                         if (m >= n) {
-                            if (ra < N) a = W.Aat(k, ra);
-                            if (ca < N) bb = W.Aat(k, ca);
+                            if (ra < N) a = W.gram_basis(k, ra);
+                            if (ca < N) bb = W.gram_basis(k, ca);
                         } else {
-                            if (ra < N) a = W.Aat(ra, k);
-                            if (ca < N) bb = W.Aat(ca, k);
+                            if (ra < N) a = W.gram_basis(ra, k);
+                            if (ca < N) bb = W.gram_basis(ca, k);
                         }
                     }
                     acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bb, acc, 0, 0, 0);
@@ -2014,7 +2040,7 @@ __device__ __forceinline__ void gram_eigs(Wave &W, double &lam_lane, int &N) {
 }
 
 // lsqnonneg_gcv! with method :brent (:1136-1205)
-__device__ __forceinline__ void reg_gcv(Wave &W, double &mu_out, double &chi2_out) {
+template <class Wv> __device__ __forceinline__ void reg_gcv(Wv &W, double &mu_out, double &chi2_out) {
     double lam;
     int N;
     {
@@ -2058,14 +2084,14 @@ __device__ __forceinline__ void reg_gcv(Wave &W, double &mu_out, double &chi2_ou
 // current state: it may only switch to a cached state no wider than the current one, and every earlier state is
 // wider, so the state cache is not kept. A voxel whose caches would still overflow gets no outputs (they stay NaN)
 // and is counted; the rest of the volume is unaffected.
-struct LCurve {
-    Wave &W;
+template <class Wv> struct LCurve {
+    Wv &W;
     gdbl *fcx, *fcP0, *fcP1;
     gdbl *pcx, *pcP0, *pcP1, *pcC;
     int nfc, npc;
     bool overflow;
 
-    __device__ __forceinline__ LCurve(Wave &w) : W(w), nfc(0), npc(0), overflow(false) {
+    __device__ __forceinline__ LCurve(Wv &w) : W(w), nfc(0), npc(0), overflow(false) {
         gdbl *p = w.lc;
         fcx = p; fcP0 = p + kLcurveCap; fcP1 = p + 2 * kLcurveCap;
         p += 3 * kLcurveCap;
@@ -2215,9 +2241,9 @@ struct LCurve {
     }
 };
 
-__device__ __forceinline__ void reg_lcurve(Wave &W, double &mu_out, double &chi2_out) {
+template <class Wv> __device__ __forceinline__ void reg_lcurve(Wv &W, double &mu_out, double &chi2_out) {
     W.cache_reset();
-    LCurve lc(W);
+    LCurve<Wv> lc(W);
     double logmu = lc.corner(-8.0, 2.0, 1e-4, 1e-4, 1e-4);
     if (lc.overflow) W.failed = true;
     double mu_final = exp(logmu);
@@ -2262,9 +2288,10 @@ __device__ __forceinline__ void hermite_minimize(double a, double b, double u0, 
     uo = uend;
 }
 
-struct FlipSearch {
-    Wave &W;
+template <class Wv> struct FlipSearch {
+    Wv &W;
     cgdbl *AsT, *dAsT;  // K column-major bases and their alpha-derivatives, column stride basis_ld(m)
+    cgdbl *As;          // the bases row-major (m x n each), for wave types that solve on them
     int K, numeval, mineval;
     unsigned long long seen;
     double al, u, du;  // lane k: grid angle, loss, gradient
@@ -2278,7 +2305,7 @@ struct FlipSearch {
         cgdbl *AT = AsT + (size_t)k * n * ldg, *dAT = dAsT + (size_t)k * n * ldg;
         int ns;
         double rn;
-        W.solve(AT, false, 0.0, ns, rn);
+        W.solve(Wv::kRowMajor ? As + (size_t)k * m * n : AT, false, 0.0, ns, rn);
         double ell = rn * rn;
         if (legacy) {  // loss! (src/splines.jl:1010-1014): no gradient
             if (W.L == k) { u = ell; du = 0.0; }
@@ -2430,11 +2457,11 @@ struct FlipSearch {
 };
 
 // Basis at one flip angle: n EPG curves, two per wave (32-lane groups) when the echo window fits.
-template <typename T>
-__device__ __forceinline__ void voxel_basis_t(Wave &W, bool general, double alpha, double beta, double E1, cgdbl *E2,
+template <typename T, class Wv>
+__device__ __forceinline__ void voxel_basis_t(Wv &W, bool general, double alpha, double beta, double E1, cgdbl *E2,
                                               gdbl *A0out) {
     const int m = W.m, n = W.n, L = W.L;
-    const int ldg = basis_ld(m);  // column-major output: column j at A0out + j * ldg
+    const int ldg = W.basis_cs(), rs = W.basis_rs();  // element (i, j) at A0out + j * ldg + i * rs
     if constexpr (std::is_same<T, double>::value) {
         if (!general) {
             // two curves per lane group and pass (epg_const_pair)
@@ -2444,12 +2471,12 @@ __device__ __forceinline__ void voxel_basis_t(Wave &W, bool general, double alph
                     const int j1 = jp + h, j2 = jp + 2 + h;
                     const int jj1 = j1 < n ? j1 : n - 1, jj2 = j2 < n ? j2 : n - 1;
                     epg_const_pair<32>(alpha, E1, E2[jj1], E2[jj2], m, s, j1 < n, j2 < n, A0out + jj1 * ldg,
-                                       A0out + jj2 * ldg, 1);
+                                       A0out + jj2 * ldg, rs);
                 }
             } else {
                 for (int j = 0; j < n; j += 2) {
                     const int j2 = j + 1 < n ? j + 1 : n - 1;
-                    epg_const_pair<64>(alpha, E1, E2[j], E2[j2], m, L, true, j + 1 < n, A0out + j * ldg, A0out + j2 * ldg, 1);
+                    epg_const_pair<64>(alpha, E1, E2[j], E2[j2], m, L, true, j + 1 < n, A0out + j * ldg, A0out + j2 * ldg, rs);
                 }
             }
             return;
@@ -2461,14 +2488,15 @@ __device__ __forceinline__ void voxel_basis_t(Wave &W, bool general, double alph
             int j = jp + h;
             bool valid = j < n;
             int jj = valid ? j : n - 1;
-            epg_curve<32, T>(general, alpha, beta, E1, E2[jj], m, s, valid, A0out + jj * ldg, nullptr, 1, nullptr);
+            epg_curve<32, T>(general, alpha, beta, E1, E2[jj], m, s, valid, A0out + jj * ldg, nullptr, rs, nullptr);
         }
     } else {
         for (int j = 0; j < n; ++j)
-            epg_curve<64, T>(general, alpha, beta, E1, E2[j], m, L, true, A0out + j * ldg, nullptr, 1, nullptr);
+            epg_curve<64, T>(general, alpha, beta, E1, E2[j], m, L, true, A0out + j * ldg, nullptr, rs, nullptr);
     }
 }
-__device__ __forceinline__ void voxel_basis(Wave &W, bool fp32, bool general, double alpha, double beta, double E1,
+template <class Wv>
+__device__ __forceinline__ void voxel_basis(Wv &W, bool fp32, bool general, double alpha, double beta, double E1,
                                             cgdbl *E2, gdbl *A0out) {
     if (fp32) voxel_basis_t<float>(W, general, alpha, beta, E1, E2, A0out);
     else voxel_basis_t<double>(W, general, alpha, beta, E1, E2, A0out);
@@ -2482,43 +2510,10 @@ __device__ __forceinline__ void voxel_basis(Wave &W, bool fp32, bool general, do
 }
 
 // ------------------------------------ the voxel kernel ------------------------------------
-// RK = Reg (0-4) + 8 for legacy = true: the legacy code is compiled only into the legacy instantiations, so the
-// others keep their register allocation.
-template <int RK>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void t2map_kernel(T2mapParams p) {
-    constexpr int REG = RK & 7;
-    constexpr bool LEGACY = (RK & 8) != 0;
-    extern __shared__ double smem[];
-    Wave W;
-    W.L = lane_id();
-    W.m = p.m;
-    W.n = p.n;
-    W.lda = p.lda;
-    W.mw = p.mw;
-    W.rl = p.rl;
-    W.gld = p.gld;
-    ldbl *s = (ldbl *)smem;
-    // every double array has an even length, so each starts 16-byte aligned
-    const int bz = (p.mw + 1) & ~1;
-    W.A = s; s += (size_t)p.n * p.lda;
-    W.b = s; s += bz;
-    W.zz = W.b;  // the warm start forms its residual there before b takes the right-hand side
-    const int ne = (p.n + 1) & ~1;
-    W.x = s; s += ne;
-    W.cmu = s; s += kTikhCache;
-    W.crn = s; s += kTikhCache;
-    W.csemi = s; s += kTikhCache;
-    W.spt = s; s += LEGACY ? kSplineKnots : 0;
-    W.spc = s; s += LEGACY ? kSplineMaxPts : 0;
-    gdbl *slot = (gdbl *)p.scratch + (int64_t)blockIdx.x * p.slot_stride;
-    // slot: the voxel's column-major basis (one copy), the L-curve caches, the Tikhonov cache solutions, the
-    // normalized signal, the final distribution and the workspace rows of the split schedule
-    W.A0s = slot;
-    W.lc = slot + (int64_t)basis_ld(p.m) * p.n;
-    W.cx = W.lc + 7 * kLcurveCap;
-    W.b0 = W.cx + (size_t)kTikhCache * p.n;  // the voxel's normalized signal
-    W.xf = W.b0 + ((p.m + 1) & ~1);           // the voxel's final distribution
-    W.G = W.xf + ne;  // workspace rows [rl, mw) of the split schedule, n columns of stride gld
+// One persistent wave: voxels from the device counter until the list is done. Shared by the memory-resident kernel
+// (Wave) and the register-resident one (RegWave).
+template <int REG, bool LEGACY, class Wv>
+__device__ __forceinline__ void t2map_voxels(const T2mapParams &p, Wv &W) {
     W.flops = 0;
     W.flops32 = 0;
     W.solves = 0;
@@ -2538,6 +2533,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         if ((int64_t)vi >= nvox) break;
         const int64_t I = ((cgi64 *)p.vox)[vi];
         W.failed = false;
+        W.begin_voxel();
+        const unsigned long long flops0 = W.flops, flops32_0 = W.flops32, solves0 = W.solves;
         // voxelwise_T2_distribution! (:201-238): normalize by the max echo
         double mx = 0.0;
         for (int i = L; i < m; i += kWave) {
@@ -2553,12 +2550,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         double alpha_v;
         if (p.mode == kModeFixed) {
             alpha_v = p.setflip;
-            W.A0 = (cgdbl *)p.Afixed;
+            W.A0 = (cgdbl *)(Wv::kRowMajor ? p.AfixedR : p.Afixed);
         } else {
             if (p.mode == kModeB1) {
                 alpha_v = p.alpha_in[I];
             } else {
-                FlipSearch fs{W, (cgdbl *)p.AsT, (cgdbl *)p.dAsT, p.K, 0, p.mineval, 0ull, 0.0, 0.0, 0.0,
+                FlipSearch<Wv> fs{W, (cgdbl *)p.AsT, (cgdbl *)p.dAsT, (cgdbl *)p.As, p.K, 0, p.mineval, 0ull, 0.0, 0.0, 0.0,
                               LEGACY, 0ull, 0.0, 0.0};
                 fs.al = (L < p.K) ? p.alphas[L] : p.alphas[p.K - 1];
                 fs.u = NAN;
@@ -2585,6 +2582,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
             reg_mdp(W, delta, muv, chi2v);
         }
         DMI_PT1(kPhRegTotal);
+        if (W.redo()) {  // the voxel goes to the list the memory-resident kernel runs next
+            if (L == 0) p.redo[atomicAdd(p.redo_count, 1u)] = I;
+            W.flops = flops0;  // counted there
+            W.flops32 = flops32_0;
+            W.solves = solves0;
+            __syncthreads();
+            continue;
+        }
         if (W.failed) {  // outputs stay as the caller filled them (NaN)
             W.nfailed += 1;
             __syncthreads();
@@ -2599,7 +2604,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         double pr2 = 0.0, prs = 0.0;
         for (int i = L; i < m; i += kWave) {
             double fit = 0.0;
-            for (int j = 0; j < n; ++j) fit += W.A0[j * basis_ld(m) + i] * W.xf[j];
+            for (int j = 0; j < n; ++j) fit += W.basis(i, j) * W.xf[j];
             double bi = W.b0[i] * max_signal;
             double res = fit - bi;
             if (i == L) res0 = res; else res1 = res;
@@ -2632,7 +2637,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         }
         if (L < n) p.dist[I + V * L] = xs;
         if (p.decaybasis && p.mode != kModeFixed && L < n)
-            for (int i = 0; i < m; ++i) p.decaybasis[I + V * (i + (int64_t)m * L)] = W.A0[L * basis_ld(m) + i];
+            for (int i = 0; i < m; ++i) p.decaybasis[I + V * (i + (int64_t)m * L)] = W.basis(i, L);
         __syncthreads();
         DMI_PT1(kPhVoxel);
     }
@@ -2645,6 +2650,82 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         if (W.status) atomicOr(p.status, W.status);
     }
 }
+
+// RK = Reg (0-4) + 8 for legacy = true: the legacy code is compiled only into the legacy instantiations, so the
+// others keep their register allocation.
+template <int RK>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void t2map_kernel(T2mapParams p) {
+    constexpr bool LEGACY = (RK & 8) != 0;
+    extern __shared__ double smem[];
+    Wave W;
+    W.L = lane_id();
+    W.m = p.m;
+    W.n = p.n;
+    W.lda = p.lda;
+    W.mw = p.mw;
+    W.rl = p.rl;
+    W.gld = p.gld;
+    ldbl *s = (ldbl *)smem;
+    // every double array has an even length, so each starts 16-byte aligned
+    const int bz = (p.mw + 1) & ~1;
+    W.A = s; s += (size_t)p.n * p.lda;
+    W.b = s; s += bz;
+    W.zz = W.b;  // the warm start forms its residual there before b takes the right-hand side
+    const int ne = (p.n + 1) & ~1;
+    W.x = s; s += ne;
+    W.cmu = s; s += kTikhCache;
+    W.crn = s; s += kTikhCache;
+    W.csemi = s; s += kTikhCache;
+    W.spt = s; s += LEGACY ? kSplineKnots : 0;
+    W.spc = s; s += LEGACY ? kSplineMaxPts : 0;
+    gdbl *slot = (gdbl *)p.scratch + (int64_t)blockIdx.x * p.slot_stride;
+    // slot: the voxel's column-major basis (one copy), the L-curve caches, the Tikhonov cache solutions, the
+    // normalized signal, the final distribution and the workspace rows of the split schedule
+    W.A0s = slot;
+    W.lc = slot + (int64_t)basis_ld(p.m) * p.n;
+    W.cx = W.lc + 7 * kLcurveCap;
+    W.b0 = W.cx + (size_t)kTikhCache * p.n;  // the voxel's normalized signal
+    W.xf = W.b0 + ((p.m + 1) & ~1);           // the voxel's final distribution
+    W.G = W.xf + ne;  // workspace rows [rl, mw) of the split schedule, n columns of stride gld
+    t2map_voxels<RK & 7, LEGACY>(p, W);
+}
+
+#if DMI_REG_S
+// The voxel kernel on register-resident solves: 256 registers a lane and at most 20 KB of LDS a workgroup, so that two
+// waves share a SIMD.
+//
+// The waves attribute is not the occupancy (256 registers a lane make it two waves per SIMD) but the limit it sets on the
+// registers the compiler allocates, 512 / waves rounded down to 8: those below the solver's bank (dmi_nnls_reg.h).
+constexpr int reg_cap_waves(int S) { return S <= 64 ? 4 : 5; }
+static_assert(Bank<DMI_REG_S>::R0 >= 512 / reg_cap_waves(DMI_REG_S) / 8 * 8, "the bank overlaps the compiler's registers");
+template <int REG, int S>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(reg_cap_waves(S), reg_cap_waves(S))))
+void t2map_reg_kernel(T2mapParams p) {
+    extern __shared__ double smem[];
+    asm volatile("" ::: "v255");
+    RegWave<S> W;
+    W.L = lane_id();
+    W.m = p.m;
+    W.n = p.n;
+    const RegLayout lay = reg_layout(p.m, p.n, REG == 2);
+    W.lds = (ldbl *)smem;
+    W.x = W.lds;
+    W.b = W.lds + lay.b;
+    W.cmu = W.lds + lay.c;
+    W.crn = W.cmu + kTikhCache;
+    W.csemi = W.crn + kTikhCache;
+    W.G = W.lds + lay.T;
+    W.spt = W.spc = nullptr;
+    // the slot of t2map_kernel without workspace rows
+    gdbl *slot = (gdbl *)p.scratch + (int64_t)blockIdx.x * p.slot_stride;
+    W.A0s = slot;
+    W.lc = slot + (int64_t)basis_ld(p.m) * p.n;
+    W.cx = W.lc + 7 * kLcurveCap;
+    W.b0 = W.cx + (size_t)kTikhCache * p.n;
+    W.xf = W.b0 + ((p.m + 1) & ~1);
+    t2map_voxels<REG, false>(p, W);
+}
+#endif
 
 // ------------------------------------ T2partSEcorr ------------------------------------
 // voxelwise_T2_parts! (src/T2partSEcorr.jl:95-138): one thread per voxel, coalesced over voxels.
@@ -2673,12 +2754,19 @@ __global__ void t2part_kernel(T2partParams p) {
 }  // namespace
 
 // ------------------------------------ host-side launchers ------------------------------------
-#if !DMI_SPLIT_TU
 #ifdef DMI_PHASE_PROFILE
-extern "C" int dmi_phase_read(unsigned long long *out) {
+// readers of this unit's counters: dmi_phase_read and so on, with the size class appended in the register-resident units
+#define DMI_CAT2(a, b) a##b
+#define DMI_CAT(a, b) DMI_CAT2(a, b)
+#if DMI_REG_S
+#define DMI_PHASE_FN(name) DMI_CAT(name##_reg, DMI_REG_S)
+#else
+#define DMI_PHASE_FN(name) name
+#endif
+extern "C" int DMI_PHASE_FN(dmi_phase_read)(unsigned long long *out) {
     return (int)hipMemcpyFromSymbol(out, HIP_SYMBOL(g_phase), sizeof(g_phase));
 }
-extern "C" int dmi_phase_reset() {
+extern "C" int DMI_PHASE_FN(dmi_phase_reset)() {
     unsigned long long z[2 * kPhCount] = {0};
     unsigned long long zt[kMaxT2 + 1] = {0};
     hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(g_tikh_rows), zt, sizeof zt);
@@ -2688,13 +2776,14 @@ extern "C" int dmi_phase_reset() {
     if (e != hipSuccess) return (int)e;
     return (int)hipMemcpyToSymbol(HIP_SYMBOL(g_phase), z, sizeof z);
 }
-extern "C" int dmi_tikh_rows_read(unsigned long long *out) {
+extern "C" int DMI_PHASE_FN(dmi_tikh_rows_read)(unsigned long long *out) {
     return (int)hipMemcpyFromSymbol(out, HIP_SYMBOL(g_tikh_rows), sizeof(g_tikh_rows));
 }
-extern "C" int dmi_eig_steps_read(unsigned long long *out) {
+extern "C" int DMI_PHASE_FN(dmi_eig_steps_read)(unsigned long long *out) {
     return (int)hipMemcpyFromSymbol(out, HIP_SYMBOL(g_eig_steps), sizeof(g_eig_steps));
 }
 #endif
+#if DMI_MAIN_TU
 int t2map_lda(int m, int n) {
     int ld = (m + n + 1) & ~1;
     return (ld % 4 == 0) ? ld + 2 : ld;
@@ -2763,7 +2852,28 @@ hipError_t launch_select(const double *image, int64_t v0, int64_t v1, double thr
     return hipGetLastError();
 }
 
-#endif  // !DMI_SPLIT_TU
+#endif  // DMI_MAIN_TU
+#if DMI_REG_S
+template <> hipError_t launch_t2map_reg<DMI_REG_S>(const T2mapParams &p, int grid, size_t lds, hipStream_t s) {
+    switch (p.reg) {
+    case 0: hipLaunchKernelGGL((t2map_reg_kernel<0, DMI_REG_S>), dim3(grid), dim3(64), lds, s, p); break;
+    case 1: hipLaunchKernelGGL((t2map_reg_kernel<1, DMI_REG_S>), dim3(grid), dim3(64), lds, s, p); break;
+    case 2: hipLaunchKernelGGL((t2map_reg_kernel<2, DMI_REG_S>), dim3(grid), dim3(64), lds, s, p); break;
+    case 3: hipLaunchKernelGGL((t2map_reg_kernel<3, DMI_REG_S>), dim3(grid), dim3(64), lds, s, p); break;
+    default: hipLaunchKernelGGL((t2map_reg_kernel<4, DMI_REG_S>), dim3(grid), dim3(64), lds, s, p); break;
+    }
+    return hipGetLastError();
+}
+template <> hipError_t t2map_reg_occupancy<DMI_REG_S>(int reg, int *blocks_per_cu, size_t lds) {
+    switch (reg) {
+    case 0: return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, t2map_reg_kernel<0, DMI_REG_S>, 64, lds);
+    case 1: return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, t2map_reg_kernel<1, DMI_REG_S>, 64, lds);
+    case 2: return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, t2map_reg_kernel<2, DMI_REG_S>, 64, lds);
+    case 3: return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, t2map_reg_kernel<3, DMI_REG_S>, 64, lds);
+    default: return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, t2map_reg_kernel<4, DMI_REG_S>, 64, lds);
+    }
+}
+#else
 using T2mapKernelFn = void (*)(T2mapParams);
 #if DMI_SPLIT_TU
 // split schedules exist for the Tikhonov-regularized methods only (lcurve, chi2, mdp)
@@ -2814,11 +2924,30 @@ hipError_t t2map_occupancy_split(int reg, int legacy, int *blocks_per_cu, size_t
 }
 #else
 hipError_t launch_t2map(const T2mapParams &p, int grid, size_t lds, hipStream_t s) {
+    switch (p.rs) {
+    case 0: break;
+    case 48: return launch_t2map_reg<48>(p, grid, lds, s);
+    case 64: return launch_t2map_reg<64>(p, grid, lds, s);
+    case 72: return launch_t2map_reg<72>(p, grid, lds, s);
+    case 80: return launch_t2map_reg<80>(p, grid, lds, s);
+    default: return hipErrorInvalidValue;
+    }
 #if !DMI_SLOT_ROWS
     if (p.rl < p.mw) return launch_t2map_split(p, grid, lds, s);
 #endif
     hipLaunchKernelGGL(t2map_kernel_for(p.reg, p.legacy), dim3(grid), dim3(64), lds, s, p);
     return hipGetLastError();
+}
+
+hipError_t t2map_occupancy_reg(int rs, int reg, int *blocks_per_cu, size_t lds) {
+    switch (rs) {
+    case 48: return t2map_reg_occupancy<48>(reg, blocks_per_cu, lds);
+    case 64: return t2map_reg_occupancy<64>(reg, blocks_per_cu, lds);
+    case 72: return t2map_reg_occupancy<72>(reg, blocks_per_cu, lds);
+    case 80: return t2map_reg_occupancy<80>(reg, blocks_per_cu, lds);
+    default: break;
+    }
+    return hipErrorInvalidValue;
 }
 
 hipError_t t2map_occupancy(int reg, int legacy, int *blocks_per_cu, size_t lds, bool split) {
@@ -2866,4 +2995,5 @@ hipError_t launch_t2part(const T2partParams &p, hipStream_t s) {
 }
 
 #endif  // DMI_SPLIT_TU
+#endif  // DMI_REG_S
 }  // namespace dmi

@@ -276,6 +276,10 @@ int bind_and_select(dmi_server *S, StreamState &st, Request *r) {
         slots = std::max(slots, (size_t)dmi::t2map_slot_doubles(m, n, gld) * std::max(c.per_cu * S->num_cu, 1));
     }
     DMI_HIP(e, st.lb.scratch.ensure(sizeof(double) * slots));
+    // and for the voxels a chunk's or a trial's register-resident launch leaves
+    int64_t most = S->cfg.chunk_voxels;
+    for (const auto &c : cands) most = std::max<int64_t>(most, 8ll * S->num_cu * c.per_cu);
+    DMI_HIP(e, st.lb.redo.ensure(sizeof(int64_t) * (size_t)most));
     DMI_HIP(e, st.lb.counter.ensure(sizeof(unsigned) * 4));
     DMI_HIP(e, st.lb.counters.ensure(sizeof(unsigned long long) * 4));
     DMI_HIP(e, st.lb.status.ensure(sizeof(int) * 4));

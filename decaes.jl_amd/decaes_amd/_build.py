@@ -18,7 +18,9 @@ PHASE_LIB = PKG / "libdecaes_amd_phase.so"
 
 # dmi_kernels_split.hip: the voxel kernel of the split schedule (dmi_kernels.hip compiled once more); the instrumented
 # build keeps both schedules in dmi_kernels.hip
-SOURCES = ["dmi_kernels.hip", "dmi_kernels_split.hip", "dmi_host.cpp", "dmi_api.cpp", "dmi_server.cpp", "dmi_synth.cpp"]
+# dmi_kernels_reg.hip: once per size class of the register-resident kernel (kRegClasses of dmi_internal.h)
+REG_CLASSES = (80, 72, 64, 48)
+SOURCES = [*(f"dmi_kernels_reg.hip:{s}" for s in REG_CLASSES), "dmi_kernels.hip", "dmi_kernels_split.hip", "dmi_host.cpp", "dmi_api.cpp", "dmi_server.cpp", "dmi_synth.cpp"]
 
 HIPCC_FLAGS = [
     "-O3", "--offload-arch=gfx950", "-fPIC", "-shared", "-std=c++17",
@@ -27,6 +29,8 @@ HIPCC_FLAGS = [
     # no packed FP32 instructions (v_pk_*_f32) anywhere in device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
+    # the register-resident kernels set the waves attribute for its register limit, not for that occupancy
+    "-Wno-pass-failed",
 ]
 
 
@@ -44,11 +48,14 @@ def build(verbose: bool = False, phase_profile: bool = False) -> Path:
     out = PHASE_LIB if phase_profile else LIB
     extra = ["-DDMI_PHASE_PROFILE"] if phase_profile else []
     for src in SOURCES:
+        src, _, rows = src.partition(":")
         if phase_profile and src == "dmi_kernels_split.hip":
             continue
-        obj = obj_dir / (src + ".o")
+        obj = obj_dir / (src + rows + ".o")
         cmd = [hipcc(), *HIPCC_FLAGS, *extra, "-c", "-I", str(REPO / "include"), "-I", str(CSRC), str(CSRC / src),
                "-o", str(obj)]
+        if rows:
+            cmd.insert(1, f"-DDMI_REG_S={rows}")
         if src.endswith(".cpp"):
             cmd = [c for c in cmd if c not in ("--offload-arch=gfx950",)]
         if verbose:

@@ -23,7 +23,7 @@ WORKLOADS = {
     "chi2": ((64, 64, 8), 32, 10e-3, 40, (10e-3, 2.0), "chi2", 32, 3),
 }
 PHASES = [(1, "construct"), (2, "apply"), (3, "trisolve"), (4, "delete"), (5, "dual"), (6, "init"), (7, "nnls"),
-          (16, " select+constr"), (18, " post-apply"), (17, " feasibility"),
+          (16, " select+constr"), (19, " swap+apply"), (18, " post-apply"), (17, " feasibility"),
           (10, "flip search"), (11, "voxel basis"), (13, "gram eigs"), (8, " gram matrix"), (9, " tridiagonal"),
           (21, " eig brackets"), (12, " sturm"), (14, "regularization"),
           (15, "reg + save")]
@@ -33,10 +33,22 @@ NPH = 24
 def run(names):
     _lib.LIB_PATH = _build.PHASE_LIB
     L = _lib.load()
-    L.dmi_phase_read.argtypes = [C.POINTER(C.c_ulonglong)]
-    L.dmi_tikh_rows_read.argtypes = [C.POINTER(C.c_ulonglong)]
-    L.dmi_eig_steps_read.argtypes = [C.POINTER(C.c_ulonglong)]
     import decaes_amd as d
+
+    # the counters of each unit: the memory-resident kernels, and one register-resident kernel per size class
+    units = [""] + [f"_reg{s}" for s in _build.REG_CLASSES]
+
+    def reset():
+        for u in units:
+            getattr(L, "dmi_phase_reset" + u)()
+
+    def read(fn, count):
+        total = [0] * count
+        for u in units:
+            buf = (C.c_ulonglong * count)()
+            getattr(L, fn + u)(buf)
+            total = [a + b for a, b in zip(total, buf)]
+        return total
 
     for wl in names:
         shape, m, TE, n, T2R, reg, K, nc = WORKLOADS[wl]
@@ -44,13 +56,12 @@ def run(names):
         opts = d.T2mapOptions.from_image(img, TE=TE, nT2=n, T2Range=T2R, Reg=reg, nRefAngles=K, Chi2Factor=1.02,
                                          Silent=True)
         d.T2mapSEcorr(img, opts)  # warm-up: grid bases and buffers
-        L.dmi_phase_reset()
+        reset()
         t = time.time()
         d.T2mapSEcorr(img, opts)
         dt = time.time() - t
         st = _lib.context().stats()
-        buf = (C.c_ulonglong * (2 * NPH))()
-        L.dmi_phase_read(buf)
+        buf = read("dmi_phase_read", 2 * NPH)
         voxel = buf[10] + buf[11] + buf[15]
         print(f"== {wl}: {shape} nTE={m} nT2={n} Reg={reg} K={K}: {nin} voxels, kernel {st['kernel_ms']:.1f} ms "
               f"({nin / st['kernel_ms'] * 1e3:.0f} voxels/s), wall {dt:.2f} s, {st['nnls_solves'] / nin:.1f} "
@@ -61,13 +72,11 @@ def run(names):
                 continue
             print(f"   {name:>15s} {buf[k] / nin:13.0f} {100 * buf[k] / max(voxel, 1):7.1f}% "
                   f"{buf[NPH + k] / nin:12.2f} {buf[k] / buf[NPH + k]:12.0f}", flush=True)
-        steps = (C.c_ulonglong * 32)()
-        L.dmi_eig_steps_read(steps)
+        steps = read("dmi_eig_steps_read", 32)
         if sum(steps):
             hist = ", ".join(f"{k}: {steps[k]}" for k in range(32) if steps[k])
             print(f"   GCV eigenvalue Laguerre steps per voxel: {hist}", flush=True)
-        rows = (C.c_ulonglong * 65)()
-        L.dmi_tikh_rows_read(rows)
+        rows = read("dmi_tikh_rows_read", 65)
         tot = sum(rows)
         if tot:
             cum, p50, p99, mx = 0, None, None, max(i for i in range(65) if rows[i])

@@ -36,9 +36,10 @@ enum { DMI_PREC_FP64 = 0, DMI_PREC_MIXED = 1 };
 
 /* Launch schedule of the voxel kernel. LDS: the whole NNLS workspace of a voxel in LDS. SPLIT: the rows beyond a
  * cutoff (Tikhonov rows appended late) in the workgroup's L2-resident global slot, so that more workgroups share a
- * CU's LDS (Tikhonov-regularized methods, when it raises the workgroups per CU). AUTO: the choice measured on the
- * first large call for these sizes and kept for the process (the all-LDS schedule until then). Every schedule
- * performs the same arithmetic: results are bit-identical. */
+ * CU's LDS (Tikhonov-regularized methods, when it raises the workgroups per CU). AUTO: the workspace in registers
+ * (nTE <= 64; nTE <= 80 unregularized) or, for longer trains and the legacy path, all in LDS; where a split schedule
+ * exists it is measured against that on the first large call for these sizes and the choice kept for the process.
+ * Every schedule performs the same arithmetic: results are bit-identical. */
 enum { DMI_SCHED_AUTO = 0, DMI_SCHED_LDS = 1, DMI_SCHED_SPLIT = 2 };
 
 /* T2mapOptions (src/types.jl:19-100). Optional reals use NaN for `nothing`. */
@@ -97,7 +98,8 @@ typedef struct {
     double total_ms;       /* device time of the whole call */
     int64_t voxels_failed; /* voxels left unwritten (NaN) because a per-voxel search cache overflowed; the L-curve
                               caches hold every point the search can visit, so this stays 0 */
-    int32_t lds_rows;      /* schedule of the last launch: workspace rows held in LDS (the rest in the global slot) */
+    int32_t lds_rows;      /* schedule of the last launch: workspace rows held in LDS (the rest in the global slot);
+                            * 0: the register-resident schedule */
     int32_t workgroups_per_cu; /* and its resident workgroups (one voxel each) per CU */
 } dmi_stats;
 
