@@ -609,6 +609,7 @@ struct Wave {
     __device__ __forceinline__ double gram_basis(int i, int j) { return Aat(i, j); }
     __device__ __forceinline__ ldbl &gram_at(int r, int c) { return A[c * lda + m + r]; }
     __device__ __forceinline__ bool redo() const { return false; }
+    __device__ __forceinline__ bool basis_const(bool, double, double, cgdbl *, gdbl *) { return false; }
     __device__ __forceinline__ void begin_voxel() {}
     // row i of column j wherever it lives (i < rl: LDS, else the global slot); per-lane rows may differ
     __device__ __forceinline__ double Aget(int i, int j) {
@@ -2498,7 +2499,8 @@ __device__ __forceinline__ void voxel_basis_t(Wv &W, bool general, double alpha,
 template <class Wv>
 __device__ __forceinline__ void voxel_basis(Wv &W, bool fp32, bool general, double alpha, double beta, double E1,
                                             cgdbl *E2, gdbl *A0out) {
-    if (fp32) voxel_basis_t<float>(W, general, alpha, beta, E1, E2, A0out);
+    if (!general && W.basis_const(fp32, alpha, E1, E2, A0out)) {
+    } else if (fp32) voxel_basis_t<float>(W, general, alpha, beta, E1, E2, A0out);
     else voxel_basis_t<double>(W, general, alpha, beta, E1, E2, A0out);
     // EPG op count of the reference's split recursion: ~13 flops per retained state per echo
     const unsigned long long f = (unsigned long long)W.n * 13ull * ((unsigned long long)W.m * W.m / 4 + W.m);

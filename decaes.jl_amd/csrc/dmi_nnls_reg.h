@@ -665,6 +665,118 @@ __device__ __attribute__((noinline)) RegSolve nnls_reg(cgdbl *A0_, cgdbl *b0_, l
     return out;
 }
 
+// The voxel's basis at a constant flip angle, row-major: epg_const's recursion on two curves per LPC-lane group, with its
+// operations in its order. A step is 10 FP operations, 4 selects that shift the phase states and 2 that push the echo
+// into a shift register: v_cndmask takes its shifted operand through DPP, so a shift and its end condition are one
+// instruction per word, and the echoes are scaled and stored once per LPC steps instead of one lane's store per step. A
+// function of its own, since inside the voxel kernel the loop reloads spilled scalar registers. Per pair of curves and
+// echo 590 cycles before, about 310 now; a 56 x 60 basis is 2% of a voxel's L-curve (4% before).
+
+// One step's shifts: F takes Fr of the lane below, Fb the lane above's Fbr, R its own value of the lane below; the lanes in
+// `first` take Fbr for F and R, those in `last` zero for Fb.
+#define DMI_SHR " wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+#define DMI_SHL " wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+__device__ __forceinline__ void shift_states(int Fr, int Fbr, int &F, int &Fb, int &R, unsigned long long first,
+                                             unsigned long long last) {
+    asm("s_mov_b64 vcc, %5\n\ts_nop 1\n\tv_cndmask_b32_dpp %0, %3, %4, vcc" DMI_SHR "v_cndmask_b32_dpp %2, %2, %4, vcc" DMI_SHR
+        "s_mov_b64 vcc, %6\n\tv_cndmask_b32_dpp %1, %4, %7, vcc" DMI_SHL
+        : "=&v"(F), "=&v"(Fb), "+v"(R) : "v"(Fr), "v"(Fbr), "s"(first), "s"(last), "v"(0) : "vcc");
+}
+__device__ __forceinline__ void shift_states(float Fr, float Fbr, float &F, float &Fb, float &R, unsigned long long first,
+                                             unsigned long long last) {
+    int f, g, r = __float_as_int(R);
+    shift_states(__float_as_int(Fr), __float_as_int(Fbr), f, g, r, first, last);
+    F = __int_as_float(f);
+    Fb = __int_as_float(g);
+    R = __int_as_float(r);
+}
+__device__ __forceinline__ void shift_states(double Fr, double Fbr, double &F, double &Fb, double &R, unsigned long long first,
+                                             unsigned long long last) {
+    int f0, f1, g0, g1, r0 = __double2loint(R), r1 = __double2hiint(R);
+    asm("s_mov_b64 vcc, %10\n\ts_nop 1\n\tv_cndmask_b32_dpp %0, %6, %8, vcc" DMI_SHR "v_cndmask_b32_dpp %1, %7, %9, vcc" DMI_SHR
+        "v_cndmask_b32_dpp %4, %4, %8, vcc" DMI_SHR "v_cndmask_b32_dpp %5, %5, %9, vcc" DMI_SHR
+        "s_mov_b64 vcc, %11\n\tv_cndmask_b32_dpp %2, %8, %12, vcc" DMI_SHL "v_cndmask_b32_dpp %3, %9, %12, vcc" DMI_SHL
+        : "=&v"(f0), "=&v"(f1), "=&v"(g0), "=&v"(g1), "+v"(r0), "+v"(r1)
+        : "v"(__double2loint(Fr)), "v"(__double2hiint(Fr)), "v"(__double2loint(Fbr)), "v"(__double2hiint(Fbr)), "s"(first),
+          "s"(last), "v"(0)
+        : "vcc");
+    F = __hiloint2double(f1, f0);
+    Fb = __hiloint2double(g1, g0);
+    R = __hiloint2double(r1, r0);
+}
+#undef DMI_SHR
+#undef DMI_SHL
+
+template <typename T, int LPC>
+__device__ __forceinline__ void basis_rows(double sn_, double cs_, double m0_, double E1, cgdbl *E2, int m, int n, gdbl *A0) {
+    using N = Num<T>;
+    constexpr int G = kWave / LPC;  // curves side by side; each lane runs two
+    const int L = lane_id(), h = L / LPC, s = L % LPC;
+    const unsigned long long first = LPC == 64 ? 1ull : 0x100000001ull, last = LPC == 64 ? 1ull << 63 : 0x8000000080000000ull;
+    const T sn = N::c(sn_), cs = N::c(cs_), m0 = N::c(m0_);
+    const double E1sq = E1 * E1;
+    const T d = cs * E1sq, zero = N::c(0.0);
+#pragma unroll 1
+    for (int jp = 0; jp < n; jp += 2 * G) {
+        int j[2];
+        T a[2], b[2], c[2], cp[2], mc[2], F[2], Fb[2], Z[2], R[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            j[q] = jp + q * G + h;
+            const double e2 = E2[min(j[q], n - 1)], E2h = (e2 * e2) / 2, E1E2 = E1 * e2;
+            a[q] = N::c(E2h);
+            b[q] = cs * E2h;
+            c[q] = sn * E1E2;
+            cp[q] = (-c[q]) / 2.0;
+            mc[q] = -c[q];
+            F[q] = N::c(s == 0 ? 1.0 : 0.0);
+            Fb[q] = Z[q] = R[q] = zero;
+        }
+#pragma unroll 1
+        for (int i0 = 0; i0 < m; i0 += LPC) {
+            const int cnt = min(LPC, m - i0), full = (i0 + cnt == m) ? cnt - 1 : cnt;
+#pragma unroll 1
+            for (int i = 0; i < full; ++i) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const T C = F[q] + Fb[q], S = F[q] - Fb[q], Cp = a[q] * C, Sp = b[q] * S;
+                    const T Fr = tfma(c[q], Z[q], Cp + Sp), Fbr = tfma(mc[q], Z[q], Cp - Sp);
+                    Z[q] = tfma(cp[q], S, d * Z[q]);
+                    shift_states(Fr, Fbr, F[q], Fb[q], R[q], first, last);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if (full < cnt) {  // the train's last echo
+                    const T C = F[q] + Fb[q], S = F[q] - Fb[q];
+                    T f, g;
+                    shift_states(zero, tfma(mc[q], Z[q], tfma(a[q], C, -(b[q] * S))), f, g, R[q], first, last);
+                }
+                // lane s holds echo i0 + cnt - 1 - s
+                if (s < cnt && j[q] < n) A0[(i0 + cnt - 1 - s) * n + j[q]] = N::val(tabs(m0 * R[q]));
+            }
+        }
+    }
+}
+__device__ __attribute__((noinline)) void basis_rows_call(int fp32, double alpha_, double E1_, cgdbl *E2_, int dims_, gdbl *A0_) {
+    const double alpha = rfl(alpha_), E1 = rfl(E1_);
+    cgdbl *E2 = rflp(E2_);
+    gdbl *A0 = rflp(A0_);
+    const int dims = rfl(dims_), m = dims & 255, n = dims >> 8;
+    // the angle in radians rounded to the recursion's type, its sine and cosine rounded once more there (tsincos)
+    const bool f32 = rfl(fp32) != 0;
+    const double al = alpha * kDeg2Rad, m0 = dsind(alpha / 2);
+    double sn, cs;
+    sincos(f32 ? (double)(float)al : al, &sn, &cs);
+    if (f32) {
+        if (m / 2 + 2 <= 32) basis_rows<float, 32>(sn, cs, m0, E1, E2, m, n, A0);
+        else basis_rows<float, 64>(sn, cs, m0, E1, E2, m, n, A0);
+    } else {
+        if (m / 2 + 2 <= 32) basis_rows<double, 32>(sn, cs, m0, E1, E2, m, n, A0);
+        else basis_rows<double, 64>(sn, cs, m0, E1, E2, m, n, A0);
+    }
+}
+
 // Wave state of the register-resident kernel, with the interface of Wave that the searches use.
 template <int S> struct RegWave {
     ldbl *lds, *x, *b, *cmu, *crn, *csemi, *G;
@@ -686,6 +798,10 @@ template <int S> struct RegWave {
     __device__ __forceinline__ ldbl &gram_at(int r, int c) { return G[c * (min(m, n) | 1) + r]; }
     __device__ __forceinline__ bool redo() const { return over; }
     __device__ __forceinline__ void begin_voxel() { over = false; }
+    __device__ __forceinline__ bool basis_const(bool fp32, double alpha, double E1, cgdbl *E2, gdbl *A0out) {
+        basis_rows_call(fp32, alpha, E1, E2, m | (n << 8), A0out);
+        return true;
+    }
 
     __device__ __forceinline__ void solve(cgdbl *A0g, bool tikh, double mu, int &nsetp, double &rnorm) {
         nsetp = 0;

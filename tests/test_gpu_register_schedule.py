@@ -24,6 +24,7 @@ CASES = [
     (81, 64, "none", False, {}),
     (47, 33, "chi2", True, dict(precision="mixed", SaveNNLSBasis=True)),
     (25, 64, "gcv", True, dict(b1=True)),
+    (61, 7, "chi2", True, dict(precision="mixed", b1=True)),
 ]
 
 
