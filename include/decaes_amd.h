@@ -131,7 +131,7 @@ int dmi_t2map_f64_device(dmi_ctx *ctx, const double *d_image, const dmi_t2map_op
 /* dmi_t2map_f64_device without any device allocation. No counterpart in the reference: it is for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Intermediate buffers (grid bases, voxel list, per-workgroup slots, counters) live in a static device array of
- * about 60 MB that each device holds for the life of the process; the caller passes inputs and outputs as for
+ * about 62 MB that each device holds for the life of the process; the caller passes inputs and outputs as for
  * dmi_t2map_f64_device. Limits: nTE <= 124, nT2 <= 64, nRefAngles <= 64 (DMI_ECAPACITY beyond); the volume is
  * processed in chunks of 262144 voxels, so its size is not limited. Every call on one device shares that array:
  * calls that overlap on one device (from several contexts or threads) race and must be serialized by the caller.
