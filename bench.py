@@ -57,7 +57,7 @@ TRAFFIC_FILE = {("c2", "fp64"): ROOT / "profiles" / "t2map_kernel_gcv_240x240x48
 
 
 def measured_traffic(workload: str, precision: str):
-    """HBM bytes per t2map_kernel launch (one step) from the committed rocprofv3 FETCH_SIZE/WRITE_SIZE passes
+    """HBM bytes per voxel-kernel launch (one step) from the committed rocprofv3 FETCH_SIZE/WRITE_SIZE passes
     (calibrated against a plain 1 GiB copy), or None when no such measurement exists for the workload."""
     import re
 
@@ -550,7 +550,9 @@ def main():
                                 "chosen_by": "autotuner (measured on the first warmup slab)"}},
         "roofline": {"bound": "fp64-valu", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS, "traffic": measured_traffic(args.workload, args.precision),
-                     "kernel": f"t2map_kernel<{dmi.api._lib.REG[w['Reg']] + (8 if w.get('legacy') else 0)}>", "kernel_ms": 1e3 * kernel_s / launches,
+                     "kernel": f"{'t2map_kernel' if stats[-1]['lds_rows'] else 't2map_reg_kernel'}"
+                               f"<{dmi.api._lib.REG[w['Reg']] + (8 if w.get('legacy') else 0)}>",
+                     "kernel_ms": 1e3 * kernel_s / launches,
                      "flops_per_launch": flops64 / launches, "fp32_tflops": flops32 / kernel_s / 1e12},
     }
     if args.precision == "mixed" and ran_all and not args.no_plain:
