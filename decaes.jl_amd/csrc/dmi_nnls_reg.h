@@ -10,6 +10,10 @@
 // once per step into registers with 16 rows in each 16-lane row (the same in all four), and every FMA takes its scalar
 // from one of them with a DPP row broadcast, at the rate of a plain FMA (measured 4.2 cycles plain, 4.4 broadcast).
 //
+// Bound by VALU issue: on the 240x240x113, 56-echo, 60-bin L-curve volume the VALU is busy 57% of the cycles (28% in the
+// memory-resident kernel), a wave waits for memory 31% of its time. That volume takes 8.7 s (20.4 s before), the
+// 240x240x48, 48-echo, 40-bin gcv volume 1.52 s (2.88 s).
+//
 // Every sum has the terms, the partial sums and the order of the memory-resident solver, so the two give the same bits.
 #pragma once
 
