@@ -352,9 +352,10 @@ int t2map_schedules(std::string &err, const dmi_t2map_opts *o, std::vector<Sched
     int rc = memory_schedules(err, o, out);
     if (rc || o->schedule != DMI_SCHED_AUTO || o->legacy) return rc;
     // Wherever a size class holds the train, registers were the faster: 240x240x4 chi2 237 ms memory-resident, 103 ms here;
-    // 240x240x6 gcv 363 and 192; 240x240 lcurve 299 and 88; 16 voxels of chi2 1.30 and 1.18. Only solves
-    // with next to no work are not (12 voxels, 4 echoes, 2 bins: 48 us, 38 in LDS). The split schedule with the most workgroups per CU, the closest of the
-    // others (lcurve 170k voxels/s against 400k in a trial), stays to be measured where there are voxels enough.
+    // 240x240x6 gcv 363 and 192; 240x240 lcurve 299 and 88; 16 voxels of chi2 1.30 and 1.18. Only solves with next to no
+    // work are not (12 voxels, 4 echoes, 2 bins: 48 us, 38 in LDS). The split schedule with the most workgroups per CU, the
+    // closest of the others (lcurve 170k voxels/s against 400k in a trial), stays to be measured where there are voxels
+    // enough.
     Schedule r = out.front();  // all rows outside the slot
     r.rs = dmi::t2map_reg_class(o->nTE, o->Reg);
     if (!r.rs) return DMI_OK;
