@@ -406,10 +406,12 @@ static int memory_schedules(std::string &err, const dmi_t2map_opts *o, std::vect
 
 namespace {
 std::mutex g_sched_mu;
-std::map<std::tuple<int, int, int, int, int, int>, Schedule> g_sched;
-std::tuple<int, int, int, int, int, int> sched_key(const dmi_t2map_opts *o) {
+// legacy calls have candidates of their own (no register-resident kernel holds the legacy code), so a choice of their own
+using SchedKey = std::tuple<int, int, int, int, int, int, int>;
+std::map<SchedKey, Schedule> g_sched;
+SchedKey sched_key(const dmi_t2map_opts *o) {
     const int K = std::isnan(o->SetFlipAngle) ? o->nRefAngles : 1;
-    return {o->nTE, o->nT2, K, o->Reg, o->precision, o->RefConAngle != 180.0};
+    return {o->nTE, o->nT2, K, o->Reg, o->precision, o->RefConAngle != 180.0, o->legacy != 0};
 }
 }  // namespace
 

@@ -2965,6 +2965,7 @@ hipError_t t2map_occupancy_split(int reg, int legacy, int *blocks_per_cu, size_t
 }
 #else
 hipError_t launch_t2map(const T2mapParams &p, int grid, size_t lds, hipStream_t s) {
+    if (p.rs && p.legacy) return hipErrorInvalidValue;  // the register-resident kernels hold no legacy code
     switch (p.rs) {
     case 0: break;
     case 48: return launch_t2map_reg<48>(p, grid, lds, s);
