@@ -31,6 +31,7 @@ struct dmi_ctx {
     dmi_host::Grids grids;
     dmi_host::LaunchBufs lb;
     double *noalloc = nullptr;  // this device's address of the static scratch (dmi_t2map_f64_device_noalloc)
+    const int *status = nullptr;  // status words of the last T2map call (dmi_last_redo_voxels)
     DevBuf vox;
     // host-array staging (FP64 working copies, FP32 transfer buffers)
     DevBuf img, ain, out[12], t2p[5];
@@ -98,6 +99,7 @@ int run_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, con
                                      sizeof(double) * m, n, hipMemcpyDeviceToDevice, c->stream));
     HIPCHECK(c, dmi::launch_fill(rb.counters, sizeof(unsigned long long) * 4, 0u, c->stream));
     HIPCHECK(c, dmi::launch_fill(rb.status, sizeof(int) * 4, 0u, c->stream));
+    c->status = rb.status;
     c->stats = dmi_stats{};
     dmi::T2mapParams p = dmi_host::t2map_params(o, rb.g, d_image, d_alpha_in, d);
     std::vector<dmi_host::Schedule> cands;
@@ -205,6 +207,7 @@ int record_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, 
                                      sizeof(double) * m, n, hipMemcpyDeviceToDevice, c->stream));
     HIPCHECK(c, dmi::launch_fill(rb.counters, sizeof(unsigned long long) * 4, 0u, c->stream));
     HIPCHECK(c, dmi::launch_fill(rb.status, sizeof(int) * 4, 0u, c->stream));
+    c->status = rb.status;
     c->stats = dmi_stats{};
     dmi::T2mapParams p = dmi_host::t2map_params(o, rb.g, d_image, d_alpha_in, d);
     dmi_host::Schedule sched;
@@ -367,6 +370,7 @@ int run_t2map_host_chunks(dmi_ctx *c, const double *image, const dmi_t2map_opts 
     } else {
         HIPCHECK(c, dmi::launch_fill(rb.counters, sizeof(unsigned long long) * 4, 0u, c->stream));
         HIPCHECK(c, dmi::launch_fill(rb.status, sizeof(int) * 4, 0u, c->stream));
+        c->status = rb.status;
     }
     rc = dmi_host::t2map_schedule(c->err, &oc, sched);
     if (rc) return rc;
@@ -624,6 +628,21 @@ const char *dmi_last_error(const dmi_ctx *c) { return c ? c->err.c_str() : g_cre
 int dmi_last_stats(const dmi_ctx *c, dmi_stats *out) {
     if (!c || !out) return DMI_EINVAL;
     *out = c->stats;
+    return DMI_OK;
+}
+
+int dmi_last_redo_voxels(dmi_ctx *c, int64_t *out) {
+    if (!c || !out) return DMI_EINVAL;
+    std::lock_guard<std::mutex> lk(c->mu);
+    DMI_ON_DEVICE(c->err, c->device);
+    int rc = no_capture(c, "dmi_last_redo_voxels");
+    if (rc) return rc;
+    int n = 0;
+    if (c->status) {
+        HIPCHECK(c, hipMemcpyAsync(&n, c->status + 1, sizeof n, hipMemcpyDeviceToHost, c->stream));
+        HIPCHECK(c, hipStreamSynchronize(c->stream));
+    }
+    *out = n;
     return DMI_OK;
 }
 

@@ -89,7 +89,7 @@ struct T2mapParams {
     int64_t slot_stride;  // doubles per slot
     double *dist, *gdn, *ggm, *gva, *fnr, *snr, *alpha, *resnorm, *decaycurve, *mu, *chi2f, *decaybasis;
     unsigned long long *counters; // [0] fp64 flops, [1] nnls solves, [2] fp32 flops
-    int *status;
+    int *status;          // [0] kStatus* flags, [1] voxels put on the redo list
 };
 
 struct T2partParams {

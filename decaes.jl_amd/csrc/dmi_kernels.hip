@@ -2585,7 +2585,10 @@ __device__ __forceinline__ void t2map_voxels(const T2mapParams &p, Wv &W) {
         }
         DMI_PT1(kPhRegTotal);
         if (W.redo()) {  // the voxel goes to the list the memory-resident kernel runs next
-            if (L == 0) p.redo[atomicAdd(p.redo_count, 1u)] = I;
+            if (L == 0) {
+                p.redo[atomicAdd(p.redo_count, 1u)] = I;
+                atomicAdd(p.status + 1, 1);
+            }
             W.flops = flops0;  // counted there
             W.flops32 = flops32_0;
             W.solves = solves0;

@@ -30,7 +30,8 @@ _dp = C.POINTER(C.c_double)
 EXPORTS = (
     "dmi_create", "dmi_destroy", "dmi_set_stream", "dmi_last_error", "dmi_t2map_f64", "dmi_t2map_f64_device",
     "dmi_epg_basis_set",
-    "dmi_t2part_f64", "dmi_t2part_f64_device", "dmi_last_stats", "dmi_synth_mse",
+    "dmi_t2part_f64", "dmi_t2part_f64_device", "dmi_last_stats", "dmi_last_redo_voxels",
+    "dmi_synth_mse",
     "dmi_t2map_f32", "dmi_t2part_f32", "dmi_t2map_f64_device_noalloc",
     "dmi_server_create", "dmi_server_destroy", "dmi_server_submit", "dmi_server_wait", "dmi_server_poll",
     "dmi_server_get_stats", "dmi_server_last_error", "dmi_server_request_error",
@@ -119,6 +120,7 @@ def load() -> C.CDLL:
         L.dmi_t2part_f64.argtypes = [vp, _dp, C.POINTER(T2partOptsC), _dp, _dp, _dp, _dp]
         L.dmi_t2part_f64_device.argtypes = [vp, vp, C.POINTER(T2partOptsC), vp, vp, vp, vp]
         L.dmi_last_stats.argtypes = [vp, C.POINTER(StatsC)]
+        L.dmi_last_redo_voxels.argtypes = [vp, C.POINTER(C.c_int64)]
         L.dmi_synth_mse.argtypes = [_dp, C.c_int64, C.c_int64, C.c_int64, C.c_int32, C.c_double, C.c_double,
                                     C.c_int32, C.c_double, C.c_uint64, C.c_int32]
         L.dmi_synth_mse.restype = C.c_int64
@@ -183,6 +185,12 @@ class Context:
         s = StatsC()
         check(load().dmi_last_stats(self.handle, C.byref(s)), self.handle)
         return {k: getattr(s, k) for k, _ in StatsC._fields_}
+
+    def redo_voxels(self) -> int:
+        """Voxels of the last call that the register-resident kernel left to the memory-resident one."""
+        n = C.c_int64()
+        check(load().dmi_last_redo_voxels(self.handle, C.byref(n)), self.handle)
+        return n.value
 
 
 _contexts: dict[int, Context] = {}

@@ -173,6 +173,12 @@ int dmi_t2part_f64_device(dmi_ctx *ctx, const double *d_dist, const dmi_t2part_o
 
 int dmi_last_stats(const dmi_ctx *ctx, dmi_stats *out);
 
+/* Voxels of the last T2map call on ctx (of its last replay, for a captured call) that outgrew the register-resident
+ * kernel and that the memory-resident kernel finished; always 0 under the other schedules. Their results are the same
+ * bits either way. Waits for ctx's stream; refused while it is captured (DMI_EINVAL). After an allocation-free call the
+ * count is the device's last such call's. */
+int dmi_last_redo_voxels(dmi_ctx *ctx, int64_t *voxels);
+
 /* ---- Request loop ----
  * A device-resident counterpart of the reference's warm server (api/decaes_server.jl:95-131, which keeps a Julia
  * process alive and runs one CLI call at a time). Requests (a T2mapSEcorr call, optionally followed by

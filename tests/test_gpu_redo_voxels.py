@@ -1,0 +1,136 @@
+"""Voxels whose NNLS workspace outgrows the register-resident kernel are finished by the memory-resident one. Images that
+are known to hold such voxels (the count is asserted) through every caller of that second launch: one device call, which
+reads the count first; a host volume of several chunks and an allocation-free volume of several chunks, which launch on
+the device's count; a captured call replayed; the request loop. Every result equals the all-LDS schedule's, bit for bit,
+the tallies too: what the first kernel did on such a voxel is not counted."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {  # nTE, nT2, voxels: L-curve solves at low mu remove many columns again
+    "56x64": (56, 64, 128),
+    "64x64": (64, 64, 512),
+}
+KEYS = ("gdn", "ggm", "gva", "fnr", "snr", "alpha", "resnorm", "decaycurve", "mu", "chi2factor")
+_packed = {}
+
+
+def _opts(dmi, shape, m, n, **kw):
+    return dmi.T2mapOptions(MatrixSize=shape, nTE=m, TE=10e-3, nT2=n, T2Range=(10e-3, 2.0), Reg="lcurve", nRefAngles=32,
+                            SaveRegParam=True, SaveResidualNorm=True, SaveDecayCurve=True, Silent=True, **kw)
+
+
+def packed(dmi, name):
+    """The voxels' image, the all-LDS results and the number of voxels that outgrow the registers."""
+    if name not in _packed:
+        m, n, P = SHAPES[name]
+        img, _ = dmi.synth_mse((P, 1, 1), m, 10e-3, ncomp=3, mask_fraction=1.0, seed=5)
+        maps, dist = dmi.T2mapSEcorr(img, _opts(dmi, (P, 1, 1), m, n, schedule="lds"))
+        ctx = dmi.context(0)
+        st = ctx.stats()
+        assert st["lds_rows"] == m + n and ctx.redo_voxels() == 0
+        dmi.T2mapSEcorr(img, _opts(dmi, (P, 1, 1), m, n))
+        assert ctx.stats()["lds_rows"] == 0
+        _packed[name] = img, maps, dist, st, ctx.redo_voxels()
+    return _packed[name]
+
+
+def _spread(img, V, at):
+    """A (V, 1, 1) volume with the packed voxels at `at`, zeros (below the threshold) elsewhere."""
+    big = np.zeros((V, 1, 1, img.shape[3]), order="F")
+    big[at, 0, 0, :] = img[:, 0, 0, :]
+    return big
+
+
+def _check(got_maps, got_dist, at, img, maps, dist):
+    assert np.array_equal(got_dist[at, 0, 0, :], dist[:, 0, 0, :], equal_nan=True)
+    for k in KEYS:
+        assert np.array_equal(got_maps[k][at, 0, 0], maps[k][:, 0, 0], equal_nan=True), k
+
+
+@pytest.mark.parametrize("name", list(SHAPES))
+def test_one_call(dmi, name):
+    m, n, P = SHAPES[name]
+    img, maps, dist, st, redo = packed(dmi, name)
+    print(f"[redo] {name}: {redo} of {P} voxels", flush=True)
+    assert 0 < redo < P
+    got, gdist = dmi.T2mapSEcorr(img, _opts(dmi, (P, 1, 1), m, n))
+    s = dmi.context(0).stats()
+    _check(got, gdist, np.arange(P), img, maps, dist)
+    for k in ("voxels", "nnls_solves", "fp64_flops", "voxels_failed"):
+        assert s[k] == st[k], k
+
+
+def test_host_volume_of_several_chunks(dmi):
+    m, n, P = SHAPES["56x64"]
+    img, maps, dist, st, redo = packed(dmi, "56x64")
+    chunk = 524288  # voxels per chunk of the host-array path
+    V = 2 * chunk + 4096
+    for copies in (1, 3):  # the voxels of one chunk only, and in every chunk
+        at = np.concatenate([np.arange(P) * 7 + 11 + c * chunk for c in range(copies)])
+        print(f"[redo] host chunks, {copies} copies", flush=True)
+        big = _spread(np.concatenate([img] * copies), V, at)
+        got, gdist = dmi.T2mapSEcorr(big, _opts(dmi, (V, 1, 1), m, n))
+        s = dmi.context(0).stats()
+        assert s["lds_rows"] == 0 and s["voxels"] == copies * P
+        assert dmi.context(0).redo_voxels() == copies * redo
+        for c in range(copies):
+            _check(got, gdist, at[c * P:(c + 1) * P], img, maps, dist)
+        assert s["nnls_solves"] == copies * st["nnls_solves"] and s["fp64_flops"] == copies * st["fp64_flops"]
+
+
+def test_allocation_free_chunks_and_replays(dmi):
+    import torch
+
+    from decaes_amd import device as D
+
+    m, n, P = SHAPES["56x64"]
+    img, maps, dist, st, redo = packed(dmi, "56x64")
+    chunk = 262144  # voxels per chunk of the allocation-free path
+    V, copies = 2 * chunk + 4096, 3
+    at = np.concatenate([np.arange(P) * 5 + 3 + c * chunk for c in range(copies)])
+    big = _spread(np.concatenate([img] * copies), V, at)
+    opts = _opts(dmi, (V, 1, 1), m, n)
+    dimg = torch.from_numpy(np.ascontiguousarray(big.transpose(3, 2, 1, 0))).to("cuda")
+    out = D.alloc_t2map_outputs(opts, device="cuda")
+    ctx = dmi.context(0)
+
+    def check():
+        host = {k: v.cpu().numpy().transpose(tuple(reversed(range(v.dim())))) for k, v in out.items()}
+        for c in range(copies):
+            _check(host, host["dist"], at[c * P:(c + 1) * P], img, maps, dist)
+        assert int(np.isfinite(host["gdn"]).sum()) == copies * P
+        assert ctx.redo_voxels() == copies * redo
+
+    print("[redo] allocation-free call", flush=True)
+    s = D.t2map_device(dimg, opts, out, noalloc=True)
+    torch.cuda.synchronize()
+    assert s["nnls_solves"] == copies * st["nnls_solves"] and s["fp64_flops"] == copies * st["fp64_flops"]
+    check()
+    g = D.capture(dimg, opts, out)
+    other = torch.linspace(0.0, 1.0, 1 << 20, dtype=torch.float64, device="cuda")
+    for r in range(3):
+        print(f"[redo] replay {r}", flush=True)
+        for t in out.values():
+            t.fill_(float("nan"))
+        other = torch.sin(other) + 0.5
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        check()
+
+
+def test_request_loop(dmi):
+    from decaes_amd.server import Server
+
+    m, n, P = SHAPES["56x64"]
+    img, maps, dist, _, redo = packed(dmi, "56x64")
+    assert redo > 0
+    print("[redo] request loop, chunks of 37 voxels", flush=True)
+    opts = _opts(dmi, (P, 1, 1), m, n)
+    with Server(max_streams=2, chunk_voxels=37) as srv:
+        for h in [srv.submit(img, opts) for _ in range(2)]:
+            got, gdist, _, info = srv.wait(h)
+            assert info["status"] == 0
+            _check(got, gdist, np.arange(P), img, maps, dist)
