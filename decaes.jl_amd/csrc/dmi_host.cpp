@@ -357,7 +357,7 @@ int t2map_schedules(std::string &err, const dmi_t2map_opts *o, std::vector<Sched
     // closest of the others (lcurve 170k voxels/s against 400k in a trial), stays to be measured where there are voxels
     // enough.
     Schedule r = out.front();  // all rows outside the slot
-    r.rs = dmi::t2map_reg_class(o->nTE, o->Reg);
+    r.rs = dmi::t2map_reg_class(o->nTE, o->nT2, o->Reg);
     if (!r.rs) return DMI_OK;
     const size_t lds = sizeof(double) * (size_t)dmi::reg_layout(o->nTE, o->nT2, o->Reg == DMI_REG_GCV).total;
     DMI_HIP(err, dmi::t2map_occupancy_reg(r.rs, o->Reg, &r.per_cu, lds));

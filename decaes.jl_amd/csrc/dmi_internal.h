@@ -153,14 +153,21 @@ hipError_t t2map_occupancy(int reg, int legacy, int *blocks_per_cu, size_t lds, 
 hipError_t launch_t2map_split(const T2mapParams &p, int grid, size_t lds, hipStream_t s);
 hipError_t t2map_occupancy_split(int reg, int legacy, int *blocks_per_cu, size_t lds);
 // the register-resident voxel kernel of size class S (kRegClasses), one unit per class from dmi_kernels_reg.hip
-// Size classes of the register-resident kernel. A Tikhonov solve's window holds the m rows and the appended rows whose
-// columns have left the active set again; it had at most 13 of those beyond m in 60,000 solves of the benchmark shapes
-// (99.9%: 11), and up to 3 registers are lost to the window's alignment, hence m + 16 rows. Solves without
-// regularization have m rows. A solve that outgrows its class sends the voxel to the memory-resident kernel.
+// Size classes of the register-resident kernel. Solves without regularization have m rows. A Tikhonov solve's window holds
+// the m rows and the appended rows whose columns have left the active set again, and up to 3 registers are lost to the
+// window's alignment; a solve that outgrows its class sends the voxel to the memory-resident kernel. Sixteen rows beyond m
+// are enough for chi2 and mdp (no voxel of 524,288 with 32, 48, 56 and 64 echoes and 40 to 64 bins outgrew them) and gcv
+// (one). The L-curve's solves at low mu remove more columns: with sixteen 9, 17 and 24 of 131,072 voxels each at 48, 56 and
+// 64 echoes did, all but two of them with more than 40 bins, with 20 or more none of 655,360. One such voxel doubles the time of
+// a call of a few hundred voxels (64 voxels of 56 x 64: 11.0 ms, 5.6 in the next class) and adds 6 ms to a 240x240 slice
+// (56 x 60: 87.0 ms, 81.1; 48 x 60: 78.8 and 74.5), so those trains take 20 where a class holds them; with up to 40
+// bins the larger class is the slower one (48 x 40: 51.3 ms, 52.4). 61 to 64 echoes keep 16 rows: their class is the largest.
 constexpr int kRegClasses[] = {48, 64, 72, 80};
-inline int t2map_reg_class(int m, int reg) {
-    for (int s : kRegClasses)
-        if (s >= m + (reg == 0 ? 0 : 16)) return s;
+inline int t2map_reg_class(int m, int n, int reg) {
+    const bool wide = reg == 1 && n > 40;  // the L-curve
+    for (int extra : {wide ? 20 : 16, 16})
+        for (int s : kRegClasses)
+            if (s >= m + (reg == 0 ? 0 : extra)) return s;
     return 0;
 }
 hipError_t t2map_occupancy_reg(int rs, int reg, int *blocks_per_cu, size_t lds);

@@ -187,8 +187,8 @@ __device__ __attribute__((noinline)) RegSolve nnls_reg(cgdbl *A0_, cgdbl *b0_, l
     constexpr int NB = 2;  // rows L and L + 64 of a vector held by row: m + n <= 128
     static_assert(S <= 80, "");
     // rows [0, R1) of the window always run, then a block of 16 and blocks of 8 as far as the window reaches (a
-    // comparison and branch cost 16 cycles, as much as one row's three FMAs)
-    constexpr int R1 = S - 32;
+    // comparison and branch cost 16 cycles, as much as one row's three FMAs); the largest class serves shorter trains too
+    constexpr int R1 = S == 80 ? 40 : S - 32;
     auto block = [](int k0) constexpr { return k0 < R1 ? 0 : k0 < R1 + 16 ? R1 : k0; };
     static_assert(S % 8 == 0 && R1 >= 8, "");
     const int L = lane_id();

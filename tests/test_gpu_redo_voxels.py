@@ -8,10 +8,9 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = {  # nTE, nT2, voxels: L-curve solves at low mu remove many columns again
-    "56x64": (56, 64, 128),
-    "64x64": (64, 64, 512),
-}
+# nTE, nT2, voxels: L-curve solves at low mu remove many columns again
+REDONE = "64x64"  # the largest size class with the least room beyond the train
+SHAPES = {"48x64": (48, 64, 2048), "56x64": (56, 64, 128), REDONE: (64, 64, 512)}
 KEYS = ("gdn", "ggm", "gva", "fnr", "snr", "alpha", "resnorm", "decaycurve", "mu", "chi2factor")
 _packed = {}
 
@@ -54,7 +53,10 @@ def test_one_call(dmi, name):
     m, n, P = SHAPES[name]
     img, maps, dist, st, redo = packed(dmi, name)
     print(f"[redo] {name}: {redo} of {P} voxels", flush=True)
-    assert 0 < redo < P
+    if name == REDONE:
+        assert 0 < redo < P
+    else:  # one voxel's second solve would take as long as the whole call: these trains get a larger class
+        assert redo == 0
     got, gdist = dmi.T2mapSEcorr(img, _opts(dmi, (P, 1, 1), m, n))
     s = dmi.context(0).stats()
     _check(got, gdist, np.arange(P), img, maps, dist)
@@ -63,8 +65,8 @@ def test_one_call(dmi, name):
 
 
 def test_host_volume_of_several_chunks(dmi):
-    m, n, P = SHAPES["56x64"]
-    img, maps, dist, st, redo = packed(dmi, "56x64")
+    m, n, P = SHAPES[REDONE]
+    img, maps, dist, st, redo = packed(dmi, REDONE)
     chunk = 524288  # voxels per chunk of the host-array path
     V = 2 * chunk + 4096
     for copies in (1, 3):  # the voxels of one chunk only, and in every chunk
@@ -85,8 +87,8 @@ def test_allocation_free_chunks_and_replays(dmi):
 
     from decaes_amd import device as D
 
-    m, n, P = SHAPES["56x64"]
-    img, maps, dist, st, redo = packed(dmi, "56x64")
+    m, n, P = SHAPES[REDONE]
+    img, maps, dist, st, redo = packed(dmi, REDONE)
     chunk = 262144  # voxels per chunk of the allocation-free path
     V, copies = 2 * chunk + 4096, 3
     at = np.concatenate([np.arange(P) * 5 + 3 + c * chunk for c in range(copies)])
@@ -124,8 +126,8 @@ def test_allocation_free_chunks_and_replays(dmi):
 def test_request_loop(dmi):
     from decaes_amd.server import Server
 
-    m, n, P = SHAPES["56x64"]
-    img, maps, dist, _, redo = packed(dmi, "56x64")
+    m, n, P = SHAPES[REDONE]
+    img, maps, dist, _, redo = packed(dmi, REDONE)
     assert redo > 0
     print("[redo] request loop, chunks of 37 voxels", flush=True)
     opts = _opts(dmi, (P, 1, 1), m, n)
