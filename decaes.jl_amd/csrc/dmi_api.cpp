@@ -29,7 +29,7 @@ struct dmi_ctx {
     std::mutex mu;
     dmi_stats stats{};
     dmi_host::Grids grids;
-    dmi_host::LaunchBufs lb;
+    DevBuf words, scratch;  // the call's CallWords and per-workgroup slots
     double *noalloc = nullptr;  // this device's address of the static scratch (dmi_t2map_f64_device_noalloc)
     const int *status = nullptr;  // status words of the last T2map call (dmi_last_redo_voxels)
     DevBuf vox;
@@ -74,16 +74,18 @@ int no_capture(dmi_ctx *c, const char *name) {
 }
 
 // Device memory one T2mapSEcorr call works in: the grids of its options, a voxel list of vox_cap entries, the
-// launch counters and the per-workgroup slots of the voxel kernel.
+// launch counters (device memory) and the per-workgroup slots of the voxel kernel.
 struct RunBufs {
     dmi_host::GridPtrs g;
     int64_t *vox, *redo;  // the voxel list, and as much room for the voxels the register-resident kernel leaves
     int64_t vox_cap;
-    unsigned *counter;
-    unsigned long long *counters;
-    int *status;
+    dmi::CallWords *words;
     double *slots;
     int64_t slot_doubles;
+
+    unsigned *counter() const { return &words->counter[0]; }
+    unsigned long long *counters() const { return &words->counters[0]; }
+    int *status() const { return &words->status[0]; }
 };
 
 // Voxel selection and the voxel kernel over [0, V) in chunks of vox_cap voxels (one chunk when the list holds the
@@ -97,9 +99,8 @@ int run_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, con
     if (fixed && o->SaveNNLSBasis)
         HIPCHECK(c, hipMemcpy2DAsync(d->decaybasis, sizeof(double) * m, rb.g.AsT, sizeof(double) * dmi::basis_ld(m),
                                      sizeof(double) * m, n, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHECK(c, dmi::launch_fill(rb.counters, sizeof(unsigned long long) * 4, 0u, c->stream));
-    HIPCHECK(c, dmi::launch_fill(rb.status, sizeof(int) * 4, 0u, c->stream));
-    c->status = rb.status;
+    HIPCHECK(c, dmi::launch_fill(rb.words, sizeof(dmi::CallWords), 0u, c->stream));
+    c->status = rb.status();
     c->stats = dmi_stats{};
     dmi::T2mapParams p = dmi_host::t2map_params(o, rb.g, d_image, d_alpha_in, d);
     std::vector<dmi_host::Schedule> cands;
@@ -117,10 +118,10 @@ int run_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, con
     int64_t last = 0;  // voxels of the last chunk's launch, whose second launch waits for its count
     for (int64_t v0 = 0; v0 < V; v0 += rb.vox_cap) {
         const int64_t v1 = std::min<int64_t>(V, v0 + rb.vox_cap);
-        HIPCHECK(c, dmi::launch_fill(rb.counter, sizeof(unsigned), 0u, c->stream));
-        HIPCHECK(c, dmi::launch_select(d_image, v0, v1, o->Threshold, rb.vox, rb.counter, c->stream));
+        if (v0) HIPCHECK(c, dmi::launch_fill(rb.counter(), sizeof(unsigned), 0u, c->stream));
+        HIPCHECK(c, dmi::launch_select(d_image, v0, v1, o->Threshold, rb.vox, rb.counter(), c->stream));
         unsigned nvox = 0;
-        HIPCHECK(c, hipMemcpyAsync(&nvox, rb.counter, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
+        HIPCHECK(c, hipMemcpyAsync(&nvox, rb.counter(), sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
         HIPCHECK(c, hipStreamSynchronize(c->stream));
         c->stats.voxels += nvox;
         if (nvox == 0) continue;
@@ -135,7 +136,7 @@ int run_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, con
                     dmi::T2mapParams ps = p;
                     dmi_host::apply_schedule(ps, s);
                     HIPCHECK(c, hipEventRecord(c->ev[1], c->stream));
-                    int rc = dmi_host::t2map_launch_raw(c->err, ps, rb.vox + done, cnt, rb.counter, rb.counters, rb.status,
+                    int rc = dmi_host::t2map_launch_raw(c->err, ps, rb.vox + done, cnt, rb.counter(), rb.counters(), rb.status(),
                                                         rb.redo, rb.slots, rb.slot_doubles, c->num_cu, c->stream);
                     if (rc) return rc;
                     HIPCHECK(c, hipEventRecord(c->ev[2], c->stream));
@@ -156,38 +157,36 @@ int run_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, con
         dmi_host::apply_schedule(p, sched);
         c->stats.lds_rows = p.rs ? 0 : std::min(p.rl, p.mw);
         c->stats.workgroups_per_cu = sched.per_cu;
-        int rc = dmi_host::t2map_launch_raw(c->err, p, rb.vox + done, nvox - done, rb.counter, rb.counters, rb.status,
+        int rc = dmi_host::t2map_launch_raw(c->err, p, rb.vox + done, nvox - done, rb.counter(), rb.counters(), rb.status(),
                                             rb.redo, rb.slots, rb.slot_doubles, c->num_cu, c->stream, v1 < V);
         if (rc) return rc;
         last = (v1 == V && p.rs) ? nvox - done : 0;
     }
-    unsigned long long cnt[4] = {0, 0, 0, 0};
-    auto finish = [&](unsigned *left) -> int {
+    dmi::CallWords got{};
+    auto finish = [&]() -> int {
         if (launched) {
             HIPCHECK(c, hipEventRecord(c->ev[2], c->stream));
-            HIPCHECK(c, hipMemcpyAsync(cnt, rb.counters, sizeof cnt, hipMemcpyDeviceToHost, c->stream));
-            if (left) HIPCHECK(c, hipMemcpyAsync(left, rb.counter + 2, sizeof *left, hipMemcpyDeviceToHost, c->stream));
+            HIPCHECK(c, hipMemcpyAsync(&got, rb.words, sizeof got, hipMemcpyDeviceToHost, c->stream));
         }
         HIPCHECK(c, hipEventRecord(c->ev[3], c->stream));
         HIPCHECK(c, hipEventSynchronize(c->ev[3]));
         return DMI_OK;
     };
     // the host reads the tallies here anyway, so the second launch is made only for voxels that need it
-    unsigned left = 0;
-    int rc1 = finish(last > 0 ? &left : nullptr);
+    int rc1 = finish();
     if (rc1) return rc1;
-    if (left) {
-        rc1 = dmi_host::t2map_launch_redo(c->err, p, last, rb.counter, rb.counters, rb.status, rb.redo, rb.slots, rb.slot_doubles,
-                                          c->num_cu, c->stream);
-        if (rc1 || (rc1 = finish(nullptr))) return rc1;
+    if (last > 0 && got.counter[2]) {
+        rc1 = dmi_host::t2map_launch_redo(c->err, p, last, rb.counter(), rb.counters(), rb.status(), rb.redo, rb.slots,
+                                          rb.slot_doubles, c->num_cu, c->stream);
+        if (rc1 || (rc1 = finish())) return rc1;
     }
     float kms = 0, tms = 0;
     if (launched) HIPCHECK(c, hipEventElapsedTime(&kms, c->ev[1], c->ev[2]));
     HIPCHECK(c, hipEventElapsedTime(&tms, c->ev[0], c->ev[3]));
-    c->stats.nnls_solves = (int64_t)cnt[1];
-    c->stats.fp64_flops = (int64_t)cnt[0];
-    c->stats.fp32_flops = (int64_t)cnt[2];
-    c->stats.voxels_failed = (int64_t)cnt[3];
+    c->stats.nnls_solves = (int64_t)got.counters[1];
+    c->stats.fp64_flops = (int64_t)got.counters[0];
+    c->stats.fp32_flops = (int64_t)got.counters[2];
+    c->stats.voxels_failed = (int64_t)got.counters[3];
     c->stats.kernel_ms = kms + tune_ms;
     c->stats.total_ms = tms;
     return DMI_OK;
@@ -205,22 +204,21 @@ int record_t2map_on(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, 
     if (!std::isnan(o->SetFlipAngle) && o->SaveNNLSBasis)
         HIPCHECK(c, hipMemcpy2DAsync(d->decaybasis, sizeof(double) * m, rb.g.AsT, sizeof(double) * dmi::basis_ld(m),
                                      sizeof(double) * m, n, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHECK(c, dmi::launch_fill(rb.counters, sizeof(unsigned long long) * 4, 0u, c->stream));
-    HIPCHECK(c, dmi::launch_fill(rb.status, sizeof(int) * 4, 0u, c->stream));
-    c->status = rb.status;
+    HIPCHECK(c, dmi::launch_fill(rb.words, sizeof(dmi::CallWords), 0u, c->stream));
+    c->status = rb.status();
     c->stats = dmi_stats{};
     dmi::T2mapParams p = dmi_host::t2map_params(o, rb.g, d_image, d_alpha_in, d);
     dmi_host::Schedule sched;
     int rc = dmi_host::t2map_schedule(c->err, o, sched);
     if (rc) return rc;
     dmi_host::apply_schedule(p, sched);
-    unsigned *count = rb.counter;
+    unsigned *count = rb.counter();
     p.nvox_dev = count;
     for (int64_t v0 = 0; v0 < V; v0 += rb.vox_cap) {
         const int64_t v1 = std::min<int64_t>(V, v0 + rb.vox_cap);
-        HIPCHECK(c, dmi::launch_fill(count, sizeof(unsigned), 0u, c->stream));
+        if (v0) HIPCHECK(c, dmi::launch_fill(count, sizeof(unsigned), 0u, c->stream));
         HIPCHECK(c, dmi::launch_select(d_image, v0, v1, o->Threshold, rb.vox, count, c->stream));
-        rc = dmi_host::t2map_launch_raw(c->err, p, rb.vox, v1 - v0, rb.counter, rb.counters, rb.status, rb.redo, rb.slots,
+        rc = dmi_host::t2map_launch_raw(c->err, p, rb.vox, v1 - v0, rb.counter(), rb.counters(), rb.status(), rb.redo, rb.slots,
                                         rb.slot_doubles, c->num_cu, c->stream);
         if (rc) return rc;
     }
@@ -241,9 +239,7 @@ int run_t2map(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, const 
     rc = c->grids.ensure(c->err, o, c->stream);
     if (rc) return rc;
     HIPCHECK(c, c->vox.ensure(2 * sizeof(int64_t) * std::max<int64_t>(V, 1)));
-    HIPCHECK(c, c->lb.counter.ensure(sizeof(unsigned) * 4));
-    HIPCHECK(c, c->lb.counters.ensure(sizeof(unsigned long long) * 4));
-    HIPCHECK(c, c->lb.status.ensure(sizeof(int) * 4));
+    HIPCHECK(c, c->words.ensure(sizeof(dmi::CallWords)));
     // slots for the largest persistent grid the voxel kernel can run with these options, under any schedule
     std::vector<dmi_host::Schedule> cands;
     rc = dmi_host::t2map_schedules(c->err, o, cands);
@@ -252,10 +248,9 @@ int run_t2map(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o, const 
     for (const auto &s : cands)
         slot_doubles = std::max<int64_t>(slot_doubles, dmi::t2map_slot_doubles(o->nTE, o->nT2, s.rl >= o->nTE + o->nT2 ? 0 : s.gld) *
                                                            std::max<int64_t>(1, std::min<int64_t>((int64_t)c->num_cu * std::max(s.per_cu, 1), V)));
-    HIPCHECK(c, c->lb.scratch.ensure(sizeof(double) * (size_t)slot_doubles));
+    HIPCHECK(c, c->scratch.ensure(sizeof(double) * (size_t)slot_doubles));
     RunBufs rb{c->grids.ptrs(), c->vox.as<int64_t>(), c->vox.as<int64_t>() + std::max<int64_t>(V, 1),
-               std::max<int64_t>(V, 1), c->lb.counter.as<unsigned>(),
-               c->lb.counters.as<unsigned long long>(), c->lb.status.as<int>(), c->lb.scratch.as<double>(), slot_doubles};
+               std::max<int64_t>(V, 1), c->words.as<dmi::CallWords>(), c->scratch.as<double>(), slot_doubles};
     return run_t2map_on(c, d_image, o, d_alpha_in, d, rb);
 }
 
@@ -289,9 +284,7 @@ int run_t2map_host_chunks(dmi_ctx *c, const double *image, const dmi_t2map_opts 
     if (!c->copy_stream) HIPCHECK(c, hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
     hipStream_t cs = c->copy_stream;
     HIPCHECK(c, c->vox.ensure(2 * sizeof(int64_t) * C));
-    HIPCHECK(c, c->lb.counter.ensure(sizeof(unsigned) * 4));
-    HIPCHECK(c, c->lb.counters.ensure(sizeof(unsigned long long) * 4));
-    HIPCHECK(c, c->lb.status.ensure(sizeof(int) * 4));
+    HIPCHECK(c, c->words.ensure(sizeof(dmi::CallWords)));
     HIPCHECK(c, c->pcnt.ensure(sizeof(unsigned) * (size_t)nch));
     // each chunk as a volume of its own; the fixed basis of SetFlipAngle is copied once at the end
     dmi_t2map_opts oc = *o;
@@ -306,15 +299,15 @@ int run_t2map_host_chunks(dmi_ctx *c, const double *image, const dmi_t2map_opts 
     for (const auto &s : cands)
         slot_doubles = std::max<int64_t>(slot_doubles, dmi::t2map_slot_doubles(m, n, s.rl >= m + n ? 0 : s.gld) *
                                                            std::max<int64_t>(1, std::min<int64_t>((int64_t)c->num_cu * std::max(s.per_cu, 1), C)));
-    HIPCHECK(c, c->lb.scratch.ensure(sizeof(double) * (size_t)slot_doubles));
+    HIPCHECK(c, c->scratch.ensure(sizeof(double) * (size_t)slot_doubles));
     for (int b = 0; b < 2; ++b) {
         HIPCHECK(c, c->pimg[b].ensure(sizeof(double) * (size_t)(C * m)));
         if (alpha_in) HIPCHECK(c, c->pain[b].ensure(sizeof(double) * (size_t)C));
         for (int i = 0; i < 12; ++i)
             if (hp[i]) HIPCHECK(c, c->pout[b][i].ensure(sizeof(double) * (size_t)(C * rows[i])));
     }
-    RunBufs rb{c->grids.ptrs(), c->vox.as<int64_t>(), c->vox.as<int64_t>() + C, C, c->lb.counter.as<unsigned>(),
-               c->lb.counters.as<unsigned long long>(), c->lb.status.as<int>(), c->lb.scratch.as<double>(), slot_doubles};
+    RunBufs rb{c->grids.ptrs(), c->vox.as<int64_t>(), c->vox.as<int64_t>() + C, C, c->words.as<dmi::CallWords>(),
+               c->scratch.as<double>(), slot_doubles};
     unsigned *cnt = c->pcnt.as<unsigned>();
     auto span = [&](int64_t k, int64_t &v0, int64_t &len) { v0 = k * C; len = std::min<int64_t>(C, V - v0); };
     // chunk k's rows between the caller's arrays (row pitch V) and staging set b (row pitch len)
@@ -368,9 +361,8 @@ int run_t2map_host_chunks(dmi_ctx *c, const double *image, const dmi_t2map_opts 
         kms0 = c->stats.kernel_ms;
         k0 = 1;
     } else {
-        HIPCHECK(c, dmi::launch_fill(rb.counters, sizeof(unsigned long long) * 4, 0u, c->stream));
-        HIPCHECK(c, dmi::launch_fill(rb.status, sizeof(int) * 4, 0u, c->stream));
-        c->status = rb.status;
+        HIPCHECK(c, dmi::launch_fill(rb.words, sizeof(dmi::CallWords), 0u, c->stream));
+        c->status = rb.status();
     }
     rc = dmi_host::t2map_schedule(c->err, &oc, sched);
     if (rc) return rc;
@@ -400,7 +392,7 @@ int run_t2map_host_chunks(dmi_ctx *c, const double *image, const dmi_t2map_opts 
             dmi_host::apply_schedule(p, sched);
             p.nvox_dev = cnt + k;
             HIPCHECK(c, dmi::launch_select(c->pimg[b].as<double>(), 0, len, o->Threshold, rb.vox, cnt + k, c->stream));
-            r = dmi_host::t2map_launch_raw(c->err, p, rb.vox, len, rb.counter, rb.counters, rb.status, rb.redo, rb.slots,
+            r = dmi_host::t2map_launch_raw(c->err, p, rb.vox, len, rb.counter(), rb.counters(), rb.status(), rb.redo, rb.slots,
                                            rb.slot_doubles, c->num_cu, c->stream);
             if (r) return r;
             HIPCHECK(c, hipEventRecord(ev.done[b], c->stream));
@@ -433,7 +425,7 @@ int run_t2map_host_chunks(dmi_ctx *c, const double *image, const dmi_t2map_opts 
     std::vector<unsigned> counts((size_t)nch, 0u);
     unsigned long long tot[4] = {0, 0, 0, 0};
     HIPCHECK(c, hipMemcpy(counts.data(), cnt, sizeof(unsigned) * (size_t)nch, hipMemcpyDeviceToHost));
-    HIPCHECK(c, hipMemcpy(tot, rb.counters, sizeof tot, hipMemcpyDeviceToHost));
+    HIPCHECK(c, hipMemcpy(tot, rb.counters(), sizeof tot, hipMemcpyDeviceToHost));
     for (int64_t k = k0; k < nch; ++k) voxels += std::min<int64_t>(counts[(size_t)k], std::min<int64_t>(C, V - k * C));
     float kms = 0, tms = 0;
     if (k0 < nch) HIPCHECK(c, hipEventElapsedTime(&kms, c->ev[1], c->ev[2]));
@@ -475,9 +467,7 @@ int run_t2map_noalloc(dmi_ctx *c, const double *d_image, const dmi_t2map_opts *o
     rb.g.dAs = rb.g.As + dmi::kNoAllocBasis;
     rb.g.AsT = rb.g.As + 2 * dmi::kNoAllocBasis;
     rb.g.dAsT = rb.g.As + 3 * dmi::kNoAllocBasis;
-    rb.counters = reinterpret_cast<unsigned long long *>(S);       // S[0, 4)
-    rb.status = reinterpret_cast<int *>(S + 4);                     // S[4, 6)
-    rb.counter = reinterpret_cast<unsigned *>(S + 6);               // S[6, 8)
+    rb.words = reinterpret_cast<dmi::CallWords *>(S);  // in the header
     rb.vox = reinterpret_cast<int64_t *>(S + dmi::kNoAllocOffVox);
     rb.redo = reinterpret_cast<int64_t *>(S + dmi::kNoAllocOffRedo);
     rb.vox_cap = dmi::kNoAllocVox;
@@ -585,8 +575,7 @@ int dmi_destroy(dmi_ctx *c) {
     dmi_host::DeviceGuard guard(c->device);
     if (c->own_stream) (void)hipStreamSynchronize(c->own_stream);
     c->grids.release();
-    c->lb.release();
-    DevBuf *bufs[] = {&c->vox, &c->img, &c->ain, &c->weights, &c->tlog, &c->f32};
+    DevBuf *bufs[] = {&c->words, &c->scratch, &c->vox, &c->img, &c->ain, &c->weights, &c->tlog, &c->f32};
     for (auto *b : bufs) b->release();
     for (auto &b : c->out) b.release();
     for (auto &b : c->t2p) b.release();

@@ -92,6 +92,16 @@ struct T2mapParams {
     int *status;          // [0] kStatus* flags, [1] voxels put on the redo list
 };
 
+// Device words of one T2map call, together so that one fill clears them and one copy reads them: the smallest calls are
+// some 20 microseconds of kernels, and a further copy to the host costs them about 10 (median of calls of 1 to 256 voxels
+// with 16 to 64 bins: 3% of the call).
+struct CallWords {
+    unsigned long long counters[4];  // T2mapParams.counters, [3] voxels without outputs
+    int status[4];                   // T2mapParams.status
+    unsigned counter[4];             // voxels selected, then the launches' own (t2map_launch_raw)
+};
+static_assert(sizeof(CallWords) == 64 && sizeof(CallWords) <= sizeof(double) * kNoAllocHeader, "");
+
 struct T2partParams {
     int n;
     int64_t V;
