@@ -2,7 +2,9 @@
 from __future__ import annotations
 
 import os
+import re
 import subprocess
+import tempfile
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -29,14 +31,55 @@ HIPCC_FLAGS = [
     # no packed FP32 instructions (v_pk_*_f32) anywhere in device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
-    # the register-resident kernels set the waves attribute for its register limit, not for that occupancy
-    "-Wno-pass-failed",
 ]
+# the register-resident kernels set the waves attribute for its register limit, not for that occupancy; their device
+# assembly is kept for check_bank
+REG_FLAGS = ["-Wno-pass-failed", "--save-temps=obj"]
 
 
 def hipcc() -> str:
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     return str(Path(rocm) / "bin" / "hipcc")
+
+
+def _vgprs(text: str) -> set[int]:
+    out = set()
+    for lo, hi, one in re.findall(r"\bv(?:\[(\d+):(\d+)\]|(\d+))(?![\w\[])", text):
+        out |= {int(one)} if one else set(range(int(lo), int(hi) + 1))
+    return out
+
+
+def check_bank(asm: str, rows: int) -> None:
+    """The register-resident solver addresses the registers from 256 - 2 rows on by name in inline assembly, which the
+    compiler does not know of, and writes its DPP reads there too, past the compiler's hazard checks. In the device
+    assembly of a size class: no instruction of the compiler's names a register of the bank, and every DPP read comes at
+    least two wait states after a VALU write of its source."""
+    bank, inline, recent = 256 - 2 * rows, False, []  # recent: registers written in each of the last two wait states
+    for no, line in enumerate(asm.splitlines(), 1):
+        if line.lstrip().startswith((";;#ASMSTART", ";;#ASMEND")):
+            inline = "ASMSTART" in line
+            continue
+        text = line.split(";")[0].strip()
+        if not text or text.startswith(".") or text.endswith(":"):
+            continue
+        op, _, args = text.replace("\t", " ").partition(" ")
+        args = [a.strip() for a in args.split(",")]
+        if not inline and max(_vgprs(text), default=0) >= bank:
+            raise RuntimeError(f"{rows}-row class: the compiler uses the solver's registers (v{bank} on) in line {no}: {text}")
+        if "_dpp" in op and any(_vgprs(args[1].split()[0]) & w for w in recent):
+            raise RuntimeError(f"{rows}-row class: a DPP read follows the write of its source too closely in line {no}: {text}")
+        states = int(args[0], 0) + 1 if op == "s_nop" else 1
+        recent = (recent + [set()] * (states - 1) + [_vgprs(args[0]) if op.startswith("v_") else set()])[-2:]
+
+
+def _compile(cmd: list[str], obj: Path, rows: str) -> None:
+    if not rows:
+        subprocess.run([*cmd, "-o", str(obj)], check=True)
+        return
+    with tempfile.TemporaryDirectory(dir=obj.parent) as tmp:
+        subprocess.run([*cmd, *REG_FLAGS, "-o", str(Path(tmp) / obj.name)], check=True)
+        check_bank(next(Path(tmp).glob("*gfx950.s")).read_text(), int(rows))
+        os.replace(Path(tmp) / obj.name, obj)
 
 
 def build(verbose: bool = False, phase_profile: bool = False) -> Path:
@@ -52,20 +95,19 @@ def build(verbose: bool = False, phase_profile: bool = False) -> Path:
         if phase_profile and src == "dmi_kernels_split.hip":
             continue
         obj = obj_dir / (src + rows + ".o")
-        cmd = [hipcc(), *HIPCC_FLAGS, *extra, "-c", "-I", str(REPO / "include"), "-I", str(CSRC), str(CSRC / src),
-               "-o", str(obj)]
+        cmd = [hipcc(), *HIPCC_FLAGS, *extra, "-c", "-I", str(REPO / "include"), "-I", str(CSRC), str(CSRC / src)]
         if rows:
             cmd.insert(1, f"-DDMI_REG_S={rows}")
         if src.endswith(".cpp"):
             cmd = [c for c in cmd if c not in ("--offload-arch=gfx950",)]
         if verbose:
             print(" ".join(cmd), flush=True)
-        cmds.append(cmd)
+        cmds.append((cmd, obj, rows))
         objs.append(str(obj))
     # the sources compile independently: one hipcc process each, at most MAX_JOBS (or the CPU count) at once
     jobs = max(1, min(len(cmds), int(os.environ.get("MAX_JOBS", 0)) or os.cpu_count() or 1))
     with ThreadPoolExecutor(jobs) as pool:
-        for f in [pool.submit(subprocess.run, cmd, check=True) for cmd in cmds]:
+        for f in [pool.submit(_compile, *c) for c in cmds]:
             f.result()
     tmp = out.with_suffix(".so.tmp")
     link = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", str(tmp), "-lpthread"]
