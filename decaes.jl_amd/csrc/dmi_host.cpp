@@ -351,11 +351,14 @@ static int memory_schedules(std::string &err, const dmi_t2map_opts *o, std::vect
 int t2map_schedules(std::string &err, const dmi_t2map_opts *o, std::vector<Schedule> &out) {
     int rc = memory_schedules(err, o, out);
     if (rc || o->schedule != DMI_SCHED_AUTO || o->legacy) return rc;
-    // Wherever a size class holds the train, registers were the faster: 240x240x4 chi2 237 ms memory-resident, 103 ms here;
-    // 240x240x6 gcv 363 and 192; 240x240 lcurve 299 and 88; 16 voxels of chi2 1.30 and 1.18. Only solves with next to no
-    // work are not (12 voxels, 4 echoes, 2 bins: 48 us, 38 in LDS). The split schedule with the most workgroups per CU, the
-    // closest of the others (lcurve 170k voxels/s against 400k in a trial), stays to be measured where there are voxels
-    // enough.
+    // Registers wherever a size class holds the train: 240x240x4 chi2 237 ms memory-resident, 103 ms here; 240x240x6 gcv 362
+    // and 192; 240x240 lcurve 299 and 82; 16 voxels of chi2 (32 x 40) 1.29 and 1.18. While every voxel has a SIMD of its own
+    // (up to 1024 of them), solves with little work are the slower ones. Kernel times of 64 voxels, against all-LDS: 1.10 to
+    // 1.27 with 2 bins; from 16 echoes on 0.91 to 1.09 with 8 bins and 0.86 to 1.06 with 16; from 32 echoes and 24 bins on
+    // 0.82 to 1.03. With 2048 voxels and more, chi2, gcv and lcurve are at 0.94 or below from 4 bins on; what stays slower is a
+    // fixed angle with one solve per voxel and few bins (none 1.08, mdp 1.2 with 8 bins). A caller with many such calls asks
+    // for schedule "lds". The split schedule with the most workgroups per CU, the closest of the others (lcurve 170k voxels/s
+    // against 400k in a trial), stays to be measured where there are voxels enough.
     Schedule r = out.front();  // all rows outside the slot
     r.rs = dmi::t2map_reg_class(o->nTE, o->nT2, o->Reg);
     if (!r.rs) return DMI_OK;

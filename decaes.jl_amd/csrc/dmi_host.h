@@ -115,7 +115,8 @@ int t2map_schedules(std::string &err, const dmi_t2map_opts *o, std::vector<Sched
 // The process-wide choice measured for these sizes and method (false if none yet).
 bool schedule_lookup(const dmi_t2map_opts *o, Schedule &s);
 void schedule_store(const dmi_t2map_opts *o, const Schedule &s);
-// The schedule a launch of these options uses: the caller's explicit choice, else the measured one, else all-LDS.
+// The schedule a launch of these options uses: the caller's explicit choice, else the measured one, else the
+// first candidate (register-resident where a size class holds the train, all-LDS otherwise).
 int t2map_schedule(std::string &err, const dmi_t2map_opts *o, Schedule &s);
 void apply_schedule(dmi::T2mapParams &p, const Schedule &s);
 
@@ -125,8 +126,10 @@ dmi::T2mapParams t2map_params(const dmi_t2map_opts *o, const GridPtrs &g, const 
                               const dmi_t2map_out *d);
 
 // Launches the voxel kernel on voxels d_vox[0, nvox) of the request in `p` (asynchronous on `s`), and after a
-// register-resident one the memory-resident kernel on the voxels that one left (none as a rule: it then ends at
-// once). Zeroes the work counters; tallies and status accumulate into lb.counters / lb.status until the caller clears them.
+// register-resident one the memory-resident kernel on the voxels that one left (unregularized solves leave none
+// and have no second launch). That takes 29 us if there are none, else at least one voxel's time at one wave per SIMD: 6 ms
+// for an L-curve voxel of 56 x 60. Zeroes the work counters; tallies and status accumulate into lb.counters / lb.status
+// until the caller clears them.
 int t2map_launch(std::string &err, dmi::T2mapParams p, const int64_t *d_vox, int64_t nvox, LaunchBufs &lb,
                  int num_cu, hipStream_t s);
 // The same launch on caller-provided device memory: `counter`, four words of which [1] (the work counter), [2] and [3]

@@ -31,7 +31,8 @@ constexpr int64_t kNoAllocHeader = 32;
 constexpr int64_t kNoAllocGrid = 3 * 64;
 constexpr int64_t kNoAllocBasis = (int64_t)kMaxAngles * kMaxT2 * kMaxEcho;   // kMaxEcho is even: basis_ld = m
 constexpr int64_t kNoAllocVox = 262144;                                      // voxels selected per chunk
-constexpr int64_t kNoAllocSlots = 5242880;                                   // 40 MiB of slots
+// 40 MiB of slots: at 56 x 60 they hold 1254 voxels, at 64 x 64 1057, of the 2048 the register-resident kernel keeps resident
+constexpr int64_t kNoAllocSlots = 5242880;
 constexpr int64_t kNoAllocOffGrid = kNoAllocHeader;
 constexpr int64_t kNoAllocOffBasis = kNoAllocOffGrid + kNoAllocGrid;
 constexpr int64_t kNoAllocOffVox = kNoAllocOffBasis + 4 * kNoAllocBasis;

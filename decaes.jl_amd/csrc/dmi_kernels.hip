@@ -2696,8 +2696,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 }
 
 #if DMI_REG_S
-// The voxel kernel on register-resident solves: 256 registers a lane and at most 20 KB of LDS a workgroup, so that two
-// waves share a SIMD.
+// The voxel kernel on register-resident solves: 256 registers a lane, so that two waves share a SIMD where the LDS
+// (reg_layout) allows 8 workgroups per CU.
 //
 // The waves attribute is not the occupancy (256 registers a lane make it two waves per SIMD) but the limit it sets on the
 // registers the compiler allocates, 512 / waves rounded down to 8: those below the solver's bank (dmi_nnls_reg.h).

@@ -4,15 +4,19 @@
 // Lane j owns column j of the workspace: rows [p, mr) (p: the active set's size, mr: the rows appended so far) are in
 // its registers a[], row r at a[r - base]. A row leaves the window when its pivot is taken: it then belongs to the
 // triangular factor and goes to LDS. Both the window (p grows with mr in the Tikhonov solves) and the factor are small:
-// the memory-resident solver (Wave) keeps (m + n) n doubles of workspace in LDS, this one n (n + 1) / 2, so two waves
-// per SIMD fit (8 workgroups per CU instead of 2 to 4). The Householder apply, whose six 16-byte LDS operations per row
-// pair bound the memory-resident solver, is three FMAs per row here: the reflector and the right-hand side are read
-// once per step into registers with 16 rows in each 16-lane row (the same in all four), and every FMA takes its scalar
-// from one of them with a DPP row broadcast, at the rate of a plain FMA (measured 4.2 cycles plain, 4.4 broadcast).
+// the memory-resident solver (Wave) keeps (m + n) n doubles of workspace in LDS, this one n (n + 1) / 2. The registers
+// allow two waves per SIMD (8 workgroups per CU; 1 to 4 memory-resident), and up to 60 bins so does the LDS: 20 KB a
+// workgroup at 60 bins, 22 KB (7 workgroups) at 64. GCV's Gram matrix takes more than the factor where m and n are both
+// large: 27 KB (6 workgroups) at 56 x 60, 35 KB (4, one wave per SIMD) at 64 x 64.
+// The Householder apply, whose six 16-byte LDS operations per row pair bound the memory-resident solver, is three FMAs
+// per row here: the reflector and the right-hand side are read once per step into registers with 16 rows in each
+// 16-lane row (the same in all four), and every FMA takes its scalar from one of them with a DPP row broadcast (one wave
+// per SIMD: 5.3 cycles, 4.2 for a plain FMA).
 //
-// Bound by VALU issue: on the 240x240x113, 56-echo, 60-bin L-curve volume the VALU is busy 57% of the cycles (28% in the
-// memory-resident kernel), a wave waits for memory 31% of its time. That volume takes 8.7 s (20.4 s before), the
-// 240x240x48, 48-echo, 40-bin gcv volume 1.52 s (2.88 s).
+// Bound by the latency of a solve's chain (dependent FP64 operations, reductions over the wave, LDS round trips), of which
+// two waves per SIMD hide a part: on the 240x240x113, 56-echo, 60-bin L-curve volume the VALU is busy 57% of the cycles (28%
+// in the memory-resident kernel), a wave issues 52% of its time, waits 31% for results and 18% for its turn to issue. That
+// volume takes 8.7 s (20.4 s memory-resident), the 240x240x48, 48-echo, 40-bin gcv volume 1.52 s (2.88 s).
 //
 // Every sum has the terms, the partial sums and the order of the memory-resident solver, so the two give the same bits.
 #pragma once
@@ -34,8 +38,9 @@ template <class P> __device__ __forceinline__ P *rflp(P *p) {
 __device__ __forceinline__ ldbl *rfll(ldbl *p) { return (ldbl *)(uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)p); }
 
 // The lane's column, rows [0, S) of the window, in the registers v[256 - 2 S] .. v[255], addressed by name: the kernels
-// that call nnls_reg are compiled for at most bank_cap(S) compiler-allocated registers (the waves-per-SIMD attribute,
-// which the called function inherits), so nothing else lives there, and declare v255 so that all 256 are theirs. Left
+// that call nnls_reg are compiled for at most 512 / reg_cap_waves(S) compiler-allocated registers (the waves-per-SIMD
+// attribute, which the called function inherits; the build reads the assembly for it), so nothing else lives there, and
+// declare v255 so that all 256 are theirs. Left
 // to the register allocator, the 72 values of a[] were copied and spilled wherever paths that shift the window meet
 // paths that do not (60 to 140 scratch accesses per step). Every access is a volatile asm statement, so all of them stay
 // in program order; none runs with lanes switched off except the dump of one lane's column.

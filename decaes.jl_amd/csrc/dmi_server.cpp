@@ -260,8 +260,8 @@ int bind_and_select(dmi_server *S, StreamState &st, Request *r) {
         DMI_HIP(e, dmi::t2map_occupancy(reg, r->o.legacy, &per_cu, lds));
         grid = std::max(grid, per_cu * S->num_cu);
     }
-    // the request's launch schedule (its explicit choice, or the one measured for these sizes, or all-LDS until the
-    // first request of these sizes has measured the candidates, see tune_schedule)
+    // the request's launch schedule (its explicit choice, or the one measured for these sizes, or the first candidate
+    // until the first large request of these sizes has measured them, see tune_schedule)
     dmi_host::Schedule sched;
     rc = dmi_host::t2map_schedule(e, &r->o, sched);
     if (rc) return rc;
@@ -307,7 +307,7 @@ int tune_schedule(dmi_server *S, StreamState &st, Request *r) {
     if (rc) return rc;
     int64_t need = 0;
     for (const auto &c : cands) need += 8ll * S->num_cu * c.per_cu;
-    if (r->nvox < 2 * need) return DMI_OK;  // too small to measure: all-LDS for this request
+    if (r->nvox < 2 * need) return DMI_OK;  // too small to measure: the first candidate for this request
     hipEvent_t e0 = nullptr, e1 = nullptr;
     DMI_HIP(e, hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) {

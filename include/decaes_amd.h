@@ -38,8 +38,9 @@ enum { DMI_PREC_FP64 = 0, DMI_PREC_MIXED = 1 };
  * cutoff (Tikhonov rows appended late) in the workgroup's L2-resident global slot, so that more workgroups share a
  * CU's LDS (Tikhonov-regularized methods, when it raises the workgroups per CU). AUTO: the workspace in registers
  * (nTE <= 64; nTE <= 80 unregularized) or, for longer trains and the legacy path, all in LDS; where a split schedule
- * exists it is measured against that on the first large call for these sizes and the choice kept for the process.
- * Every schedule performs the same arithmetic: results are bit-identical. */
+ * exists it is measured against that on the first large call for these sizes and the choice kept for the process
+ * (legacy and plain calls each have their own). Every schedule performs the same arithmetic: results are
+ * bit-identical. */
 enum { DMI_SCHED_AUTO = 0, DMI_SCHED_LDS = 1, DMI_SCHED_SPLIT = 2 };
 
 /* T2mapOptions (src/types.jl:19-100). Optional reals use NaN for `nothing`. */
